@@ -145,6 +145,15 @@ def _ids(count, seed):
     return torch.randint(0, VOCAB, (count,), generator=_gen(seed + 7), device="cuda", dtype=torch.int32)
 
 
+class _Arena:
+    """A session's K/V cache as torch reads a foreign array; the tensor holds this, and this the session."""
+
+    def __init__(self, session):
+        self.session = session
+        self.__cuda_array_interface__ = {"shape": (LAYERS, 2, HEADS, CTX, HD), "typestr": "<f2", "strides": None,
+                                         "data": (session.kv.kv.data, False), "version": 2}
+
+
 class _Session:
     """A program's model: fp16 weights on the GPU (INT8 trunk attached for "int8"), scratch, K/V cache."""
 
@@ -161,11 +170,9 @@ class _Session:
         self.graph = None
 
     def cache(self, rows):
-        """The first `rows` positions of the cache as a tensor [layer, K|V, head, rows, 64]."""
-        shape = (LAYERS, 2, HEADS, CTX, HD)
-        face = {"shape": shape, "typestr": "<f2", "data": (self.kv.kv.data, False), "version": 2, "strides": None}
-        holder = type("Arena", (), {"__cuda_array_interface__": face})()
-        return torch.as_tensor(holder, device="cuda")[:, :, :, :rows]
+        """The first `rows` positions of the cache as a tensor [layer, K|V, head, rows, 64], which keeps the
+        session, and with it the cache, while it is held."""
+        return torch.as_tensor(_Arena(self), device="cuda")[:, :, :, :rows]
 
     def prefill(self, ids, caps=None):
         self.lib.gpt2_prefill_fill_cache(self.backend, C.byref(self.model.gpu), C.byref(self.kv.kv), ids.data_ptr(),
