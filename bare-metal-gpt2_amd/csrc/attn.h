@@ -1,5 +1,10 @@
-// attn.h -- causal attention helpers shared by the prefill / decode attention kernels and the
-// persistent decode step (one wave attends one query over a key range, online softmax).
+// attn.h -- single-query attention over the K/V cache, shared by the decode attention kernels (ops.hip,
+// decode_step.hip).
+//
+// A wave holds up to 8 NT keys: key slot s = lane / 8 of step t is key 8 t + s, and lane l of the slot
+// holds dims 8 (l & 7) .. + 7 of the key and of its value, so one load instruction reads eight whole
+// 128-byte rows of the cache.  (A lane per key, reading its own row 16 bytes at a time, touches 64 rows
+// per instruction and every row again by the next seven.)
 #pragma once
 
 #include <cmath>
@@ -8,82 +13,61 @@
 
 namespace g2 {
 
-// One wave attends one query (64 dims) over keys [j0, j1) of one head.  Keys are rows
-// `kbase + j*stride`, values `vbase + j*stride` (halves).  Scores: lane = key inside a 64-key chunk,
-// each lane reading its own 128-byte key row (64 consecutive rows = contiguous bytes in the cache).
-// Context: lane = (key slot l>>3, dim group l&7): eight lanes read one 128-byte value row with
-// 16-byte loads, so one load instruction covers 8 keys; every lane accumulates 8 dims over its key
-// slot, and the 8 slots are summed once at the end.  Online softmax across chunks (m, l, c[8]).
-// Row jcur (if any) is read from kcur / vcur instead of the strided rows: the decode step's own key
-// and value, taken straight from its qkv row while the cache copy is being written.
-struct AttnState {
-    float m, l, c[8];
-};
-
-__device__ __forceinline__ void attend_range(const f16x8 (&q)[8], const uint16_t *__restrict__ kbase,
-                                             const uint16_t *__restrict__ vbase, long stride, int j0, int j1,
-                                             float scale, AttnState &st, int jcur = -1,
-                                             const uint16_t *kcur = nullptr, const uint16_t *vcur = nullptr) {
-    const int lane = threadIdx.x & 63;
-    const int slot = lane >> 3, dg = (lane & 7) * 8;
-    for (int jc = j0; jc < j1; jc += 64) {
-        const int j = jc + lane;
-        float s = -INFINITY;
-        if (j < j1) {
-            const uint16_t *kr = (j == jcur) ? kcur : kbase + (size_t)j * stride;
-            float dot = 0.f;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const f16x8 kk = *reinterpret_cast<const f16x8 *>(kr + 8 * c);
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    dot = __builtin_amdgcn_fdot2(f16x2{q[c][2 * t], q[c][2 * t + 1]}, f16x2{kk[2 * t], kk[2 * t + 1]},
-                                                 dot, false);
-            }
-            s = dot * scale;
-        }
-        const float mnew = fmaxf(st.m, wave_max(s));   // finite: key jc < j1 is in range
-        const float p = (j < j1) ? __expf(s - mnew) : 0.f;
-        const float corr = __expf(st.m - mnew);         // st.m = -inf on the first chunk -> 0
-        st.l = st.l * corr + wave_sum(p);
-        st.m = mnew;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) st.c[e] *= corr;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int kidx = slot + 8 * t;              // key index inside the chunk
-            const float pj = __shfl(p, kidx, 64);
-            const int key = jc + kidx;
-            if (key < j1) {
-                const uint16_t *vr = (key == jcur) ? vcur : vbase + (size_t)key * stride;
-                const f16x8 vv = *reinterpret_cast<const f16x8 *>(vr + dg);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) st.c[e] += pj * (float)vv[e];
-            }
-        }
-    }
+// A value from the lane eight further on (mod 16) of the same 16-lane row: the row's other key slot.
+__device__ __forceinline__ float other_slot(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true));   // row_ror:8
 }
 
-// Sum the context over the 8 key slots; lanes 0..7 then hold dims 8*lane .. 8*lane+7.
-__device__ __forceinline__ void reduce_slots(AttnState &st) {
+// q . k / 8 of the lane's key slot, the eight lanes' parts summed (every lane of the slot gets it); -inf
+// where the slot holds no key (`on` false).
+__device__ __forceinline__ float key_score(const f16x8 q, const f16x8 k, bool on) {
+    float d = __builtin_amdgcn_fdot2(f16x2{q[0], q[1]}, f16x2{k[0], k[1]}, 0.f, false);
+    d = __builtin_amdgcn_fdot2(f16x2{q[2], q[3]}, f16x2{k[2], k[3]}, d, false);
+    d = __builtin_amdgcn_fdot2(f16x2{q[4], q[5]}, f16x2{k[4], k[5]}, d, false);
+    d = __builtin_amdgcn_fdot2(f16x2{q[6], q[7]}, f16x2{k[6], k[7]}, d, false);
+    // quad_perm xor 1, xor 2, then the other quad of the eight (row_half_mirror)
+    d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0xB1, 0xF, 0xF, true));
+    d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x4E, 0xF, 0xF, true));
+    d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x141, 0xF, 0xF, true));
+    return on ? d * 0.125f : -INFINITY;
+}
+
+// The softmax weights of a wave's scores against their maximum m, in place, and their sum l (both the
+// same in every lane).  At least one score is finite.
+template <int NT>
+__device__ __forceinline__ void key_softmax(float (&s)[NT], float &m, float &l) {
+    float mx = s[0];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        st.c[e] += __shfl_xor(st.c[e], 8, 64);
-        st.c[e] += __shfl_xor(st.c[e], 16, 64);
-        st.c[e] += __shfl_xor(st.c[e], 32, 64);
+    for (int t = 1; t < NT; ++t) mx = fmaxf(mx, s[t]);
+    mx = fmaxf(mx, other_slot(mx));
+    m = fmaxf(fmaxf(lane_f(mx, 0), lane_f(mx, 16)), fmaxf(lane_f(mx, 32), lane_f(mx, 48)));
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        s[t] = __expf(s[t] - m);
+        sum += s[t];
     }
+    sum += other_slot(sum);
+    l = cross_rows_sum(sum);
+}
+
+// c += p v on the lane's eight dims; a slot without a key adds nothing, whatever v holds.
+__device__ __forceinline__ void add_value(float (&c)[8], float p, const f16x8 v, bool on) {
+    const i32x4 b = __builtin_bit_cast(i32x4, v);
+    const f16x8 u = __builtin_bit_cast(f16x8, i32x4{on ? b[0] : 0, on ? b[1] : 0, on ? b[2] : 0, on ? b[3] : 0});
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c[e] = __builtin_fmaf(p, (float)u[e], c[e]);
+}
+
+// Sum over the wave's eight key slots: every lane ends with dims 8 (lane & 7) .. + 7.
+__device__ __forceinline__ void reduce_values(float (&c)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c[e] = group_sum(c[e] + other_slot(c[e]));
 }
 
 __device__ __forceinline__ void load_q(f16x8 (&q)[8], const uint16_t *qp) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) q[c] = *reinterpret_cast<const f16x8 *>(qp + 8 * c);
-}
-
-__device__ __forceinline__ void init_state(AttnState &st) {
-    st.m = -INFINITY;
-    st.l = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) st.c[e] = 0.f;
 }
 
 }  // namespace g2

@@ -44,21 +44,6 @@ constexpr int AP_RV = 160;                     // bytes per V row in LDS (64 dim
 // below 2^-126 may flush to zero, which is below anything an fp16 probability can hold).
 __device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Maximum over the four lane groups of a query (lanes l, l^16, l^32, l^48), on the VALU lane
-// swaps of gfx950: swapping a value with itself pairs each lane with its partner in either order.
-__device__ __forceinline__ float group_max(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float group_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // gfx950's transposing LDS read of 8 bytes (ds_read_b64_tr_b16): within each 16 lanes, lane 4k+a
 // supplies the address of 4 consecutive halves, and lane 4a+b receives half b of the addresses of
 // lanes a, 4+a, 8+a, 12+a, in that order (layout checked on the GPU).

@@ -115,8 +115,7 @@ __device__ __forceinline__ uint16_t f2h(float f) {
 // bit: the fp32 operations are written out (explicit fma) and each output is pinned in fp32 before
 // its conversion, so no kernel can fold the conversion into the fma (v_fma_mix: one rounding
 // instead of two) where another does not.
-__device__ __forceinline__ void ln_row768(const f16x4 (&x)[3], const f16x4 (&g)[3], const f16x4 (&b)[3],
-                                          f16x4 (&o)[3]) {
+__device__ __forceinline__ void ln_stats768(const f16x4 (&x)[3], float &mean, float &rstd) {
     float v[12];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -125,22 +124,30 @@ __device__ __forceinline__ void ln_row768(const f16x4 (&x)[3], const f16x4 (&g)[
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < 12; ++i) s += v[i];
-    const float mean = wave_sum(s) / (float)GPT2_N_EMBD;
+    mean = wave_sum(s) / (float)GPT2_N_EMBD;
     float q = 0.f;
 #pragma unroll
     for (int i = 0; i < 12; ++i) {
         const float d = v[i] - mean;
         q = __builtin_fmaf(d, d, q);
     }
-    const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)GPT2_N_EMBD + GPT2_LN_EPS);
+    rstd = 1.0f / sqrtf(wave_sum(q) / (float)GPT2_N_EMBD + GPT2_LN_EPS);
+}
+__device__ __forceinline__ void ln_apply768(const f16x4 &x, float mean, float rstd, const f16x4 &g, const f16x4 &b,
+                                            f16x4 &o) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+    for (int c = 0; c < 4; ++c) {
+        float y = __builtin_fmaf(((float)x[c] - mean) * rstd, (float)g[c], (float)b[c]);
+        asm volatile("" : "+v"(y));
+        o[c] = (f16)y;
+    }
+}
+__device__ __forceinline__ void ln_row768(const f16x4 (&x)[3], const f16x4 (&g)[3], const f16x4 (&b)[3],
+                                          f16x4 (&o)[3]) {
+    float mean, rstd;
+    ln_stats768(x, mean, rstd);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            float y = __builtin_fmaf((v[4 * i + c] - mean) * rstd, (float)g[i][c], (float)b[i][c]);
-            asm volatile("" : "+v"(y));
-            o[i][c] = (f16)y;
-        }
+    for (int i = 0; i < 3; ++i) ln_apply768(x[i], mean, rstd, g[i], b[i], o[i]);
 }
 
 // ln_row768 on R rows at once (row r in x[r], lane layout as above): each row goes through exactly
@@ -287,6 +294,49 @@ __device__ __forceinline__ f16x8 i8x8_to_f16x8(uint2 w) {
     i8x4_to_f16x4(w.y, h[2], h[3]);
     const i32x4 v = {(int)h[0], (int)h[1], (int)h[2], (int)h[3]};
     return __builtin_bit_cast(f16x8, v);
+}
+
+// Eight fp16 weights (one 16-byte chunk of a row) against eight fp16 x values.
+__device__ __forceinline__ float dot8(const i32x4 w, const f16x8 x, float acc) {
+    const f16x8 wh = __builtin_bit_cast(f16x8, w);
+    acc = __builtin_amdgcn_fdot2(f16x2{wh[0], wh[1]}, f16x2{x[0], x[1]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(f16x2{wh[2], wh[3]}, f16x2{x[2], x[3]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(f16x2{wh[4], wh[5]}, f16x2{x[4], x[5]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(f16x2{wh[6], wh[7]}, f16x2{x[6], x[7]}, acc, false);
+    return acc;
+}
+
+// 16 int8 codes against 16 fp16 x values (two f16x8).
+__device__ __forceinline__ float dot16q(const i32x4 w, const f16x8 x0, const f16x8 x1, float acc) {
+    f16x2 a, b;
+    i8x4_to_f16x4_v((uint32_t)w.x, a, b);
+    acc = __builtin_amdgcn_fdot2(a, f16x2{x0[0], x0[1]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(b, f16x2{x0[2], x0[3]}, acc, false);
+    i8x4_to_f16x4_v((uint32_t)w.y, a, b);
+    acc = __builtin_amdgcn_fdot2(a, f16x2{x0[4], x0[5]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(b, f16x2{x0[6], x0[7]}, acc, false);
+    i8x4_to_f16x4_v((uint32_t)w.z, a, b);
+    acc = __builtin_amdgcn_fdot2(a, f16x2{x1[0], x1[1]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(b, f16x2{x1[2], x1[3]}, acc, false);
+    i8x4_to_f16x4_v((uint32_t)w.w, a, b);
+    acc = __builtin_amdgcn_fdot2(a, f16x2{x1[4], x1[5]}, acc, false);
+    acc = __builtin_amdgcn_fdot2(b, f16x2{x1[6], x1[7]}, acc, false);
+    return acc;
+}
+
+// Maximum / sum over the four lanes l, l^16, l^32, l^48, on the VALU lane swaps of gfx950: swapping a
+// value with itself pairs each lane with its partner in either order.
+__device__ __forceinline__ float group_max(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float group_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
 // Work-group barrier for LDS traffic: waits for this wave's LDS (and scalar) operations only, not for

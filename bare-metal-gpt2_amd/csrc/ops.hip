@@ -190,81 +190,84 @@ __global__ void k_add8(f16x8 *__restrict__ x, const f16x8 *__restrict__ y, size_
     x[i] = a;
 }
 
-// Merge the NW waves' partial (m, l, c) states of one head through LDS and write the context.
-template <int NW>
-__device__ __forceinline__ void merge_waves(const AttnState &st, uint16_t *__restrict__ out) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __shared__ float sm[NW], sl[NW], sc[NW][GPT2_HEAD_DIM];
-    if (lane == 0) {
-        sm[w] = st.m;
-        sl[w] = st.l;
-    }
-    if (lane < 8) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sc[w][8 * lane + e] = st.c[e];
-    }
-    __syncthreads();
-    if (w == 0) {
-        float mx = -INFINITY;
-        for (int i = 0; i < NW; ++i) mx = fmaxf(mx, sm[i]);
-        float L = 0.f, c = 0.f;
-        for (int i = 0; i < NW; ++i) {
-            if (sl[i] == 0.f) continue;   // wave had no keys
-            const float f = __expf(sm[i] - mx);
-            L += sl[i] * f;
-            c += sc[i][lane] * f;
-        }
-        out[lane] = f2h(c / L);
-    }
-}
-
-// Decode: one work-group per head, NW waves split the keys [0, len); partial (m, l, c) states are
-// merged through LDS.  len = pos + 1 comes from the step argument.
+// Decode attention: one work-group per head, NW waves split the keys [0, len) (attn.h's layout, 64 keys
+// a wave and pass; a cache of 1024 positions is one pass), every load of a pass issued before its first
+// use; the waves' (m, l, c) states meet in LDS.  Bound by latency: a head's 256 KB of keys and values at
+// 1000 positions come through one CU.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_attn_decode(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
                                                          const uint16_t *__restrict__ Kc, const uint16_t *__restrict__ Vc,
                                                          int maxT, StepArg st_arg, int len_imm) {
-    constexpr int D = GPT2_HEAD_DIM;
-    const int w = threadIdx.x >> 6, h = blockIdx.x;
+    constexpr int D = GPT2_HEAD_DIM, NT = 8;
+    __shared__ float sm[NW], sl[NW], sc[NW][D];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = blockIdx.x;
+    const int slot = lane >> 3, dg = (lane & 7) * 8;
     const int len = min(len_imm > 0 ? len_imm : st_arg.p() + 1, maxT);
     const int per = ((len + NW - 1) / NW + 7) & ~7;   // keys per wave (multiple of 8)
     const int j0 = min(len, w * per), j1 = min(len, j0 + per);
-    f16x8 q[8];
-    load_q(q, qkv + h * D);
-    AttnState st;
-    init_state(st);
-    const uint16_t *kb = Kc + (size_t)h * maxT * D, *vb = Vc + (size_t)h * maxT * D;
-    if (j0 < j1) attend_range(q, kb, vb, D, j0, j1, 0.125f, st);
-    reduce_slots(st);
-    merge_waves<NW>(st, att + h * D);
-}
-
-// Decode step, fused: appends this position's K and V (head h's 64 values of each) to the cache and
-// attends over [0, pos], reading key/value pos from the qkv row itself.
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_attn_decode_append(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
-                                                                uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc,
-                                                                int maxT, StepArg st_arg) {
-    constexpr int E = GPT2_N_EMBD, D = GPT2_HEAD_DIM;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = blockIdx.x;
-    const int pos = st_arg.p();
-    if ((unsigned)pos >= (unsigned)maxT) return;   // uniform over the grid: nothing to attend
-    const size_t hoff = (size_t)h * maxT * D;
-    if (w == 0) {
-        Kc[hoff + (size_t)pos * D + lane] = qkv[E + h * D + lane];
-        Vc[hoff + (size_t)pos * D + lane] = qkv[2 * E + h * D + lane];
+    const uint16_t *kb = Kc + (size_t)h * maxT * D + dg, *vb = Vc + (size_t)h * maxT * D + dg;
+    const f16x8 q = *reinterpret_cast<const f16x8 *>(qkv + h * D + dg);
+    float m = -INFINITY, l = 0.f, c[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int jc = j0; jc < j1; jc += 8 * NT) {
+        const int nt = (min(8 * NT, j1 - jc) + 7) >> 3;   // wave-uniform
+        f16x8 kr[NT], vr[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if (t < nt) kr[t] = *reinterpret_cast<const f16x8 *>(kb + (size_t)min(jc + slot + 8 * t, j1 - 1) * D);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if (t < nt) vr[t] = *reinterpret_cast<const f16x8 *>(vb + (size_t)min(jc + slot + 8 * t, j1 - 1) * D);
+        float s[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            s[t] = -INFINITY;
+            if (t < nt) s[t] = key_score(q, kr[t], jc + slot + 8 * t < j1);
+        }
+        float mc, lc;
+        key_softmax<NT>(s, mc, lc);
+        if (jc > j0) {   // a cache longer than one pass: this pass joins the earlier ones
+            const float mn = fmaxf(m, mc), fo = __expf(m - mn), fc = __expf(mc - mn);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c[e] *= fo;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) s[t] *= fc;
+            l = l * fo + lc * fc;
+            m = mn;
+        } else {
+            m = mc;
+            l = lc;
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if (t < nt) add_value(c, s[t], vr[t], jc + slot + 8 * t < j1);
     }
-    const int len = pos + 1;
-    const int per = ((len + NW - 1) / NW + 7) & ~7;   // keys per wave (multiple of 8)
-    const int j0 = min(len, w * per), j1 = min(len, j0 + per);
-    f16x8 q[8];
-    load_q(q, qkv + h * D);
-    AttnState st;
-    init_state(st);
-    if (j0 < j1)
-        attend_range(q, Kc + hoff, Vc + hoff, D, j0, j1, 0.125f, st, pos, qkv + E + h * D, qkv + 2 * E + h * D);
-    reduce_slots(st);
-    merge_waves<NW>(st, att + h * D);
+    reduce_values(c);
+    if (lane == 0) {
+        sm[w] = m;
+        sl[w] = l;
+    }
+    if (lane < 8) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc[w][8 * lane + e] = c[e];
+    }
+    __syncthreads();
+    if (w == 0) {
+        float mw[NW], lw[NW], mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            mw[i] = sm[i];
+            lw[i] = sl[i];
+            mx = lw[i] != 0.f ? fmaxf(mx, mw[i]) : mx;
+        }
+        float L = 0.f, o = 0.f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const float f = lw[i] != 0.f ? __expf(mw[i] - mx) : 0.f;   // 0: the wave had no keys
+            L += lw[i] * f;
+            o += sc[i][lane] * f;
+        }
+        att[h * D + lane] = f2h(o / L);
+    }
 }
 
 // ------------------------------------------------------------------ KV cache writes
@@ -367,11 +370,6 @@ void attn_decode(uint16_t *att, const uint16_t *qkv, const uint16_t *K, const ui
                  int len_imm) {
     hipLaunchKernelGGL(k_attn_decode<16>, dim3(GPT2_N_HEAD), dim3(1024), 0, stream(), att, qkv, K, V, maxT, st, len_imm);
     check_launch("k_attn_decode");
-}
-
-void attn_decode_append(uint16_t *att, const uint16_t *qkv, uint16_t *K, uint16_t *V, int maxT, StepArg st) {
-    hipLaunchKernelGGL(k_attn_decode_append<16>, dim3(GPT2_N_HEAD), dim3(1024), 0, stream(), att, qkv, K, V, maxT, st);
-    check_launch("k_attn_decode_append");
 }
 
 void argmax_advance(const uint16_t *logits, int V, int *state, int *tokens, int max_pos) {

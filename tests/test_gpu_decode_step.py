@@ -1,0 +1,111 @@
+"""The multi-kernel decode step's kernels (csrc/decode_step.hip) against the general sequence (one launch
+per op through the backend's slots), and decode attention against float64 attention.
+
+A step takes the general sequence when a buffer is not 16-byte aligned; a copy of one LayerNorm gain at an
+odd address makes the same weights take it.  Both round to fp16 at the same points and differ in the order
+of fp32 sums, so logits and cache rows are held to the gates of the persistent step against the
+eager one: rel_err = max|a - b| / max|b| <= 1e-2, KL < 2e-3."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+V, E, H, D, MAXT = 50257, 768, 12, 64, 1024
+
+
+@pytest.fixture(scope="module")
+def model(pkg, synth):
+    m = pkg.Model(synth.make_body(seed=77, plain=False))
+    yield m
+    m.free()
+
+
+def random_cache(pkg, L, kv, pos, seed):
+    """Rows [0, pos) ordinary keys and values; every later row NaN, which no step may read."""
+    c = np.full((12, 2, H, MAXT, D), 0x7E00, np.uint16)
+    c[:, :, :, :pos] = np.random.default_rng(seed).standard_normal((12, 2, H, pos, D), dtype=np.float32).astype(np.float16).view(np.uint16)
+    assert L.gpt2_h2d(kv.kv.data, c.ctypes.data, c.nbytes) == 0
+    kv.kv.len = pos
+
+
+def step(pkg, L, gpu, kv, scr, backend, token, pos):
+    logits, caps = pkg.Dev(V * 2), pkg.Dev(14 * E * 2)
+    L.gpt2_decode_step_cuda(pkg.backend(backend), C.byref(gpu), C.byref(kv.kv), token, pos, C.byref(scr.s), logits.ptr, caps.ptr)
+    L.gpt2_sync()
+    pkg.check("decode step")
+    assert kv.kv.len == pos + 1
+    cache = np.empty((12, 2, H, MAXT, D), np.uint16)
+    assert L.gpt2_d2h(cache.ctypes.data, kv.kv.data, cache.nbytes) == 0
+    return (oracle.f16_to_f32(logits.numpy(np.uint16, (V,))), oracle.f16_to_f32(caps.numpy(np.uint16, (14, E))), cache)
+
+
+def rel_err(a, b):
+    return float(np.abs(a.astype(np.float64) - b).max() / np.abs(b).max())
+
+
+@pytest.mark.parametrize("backend,keep", [("gemv", None), ("int8", None), ("int8", 0), ("int8", 3)])
+def test_step_matches_general_sequence(pkg, L, model, backend, keep):
+    """Positions at the edges of the key splits, waves and passes; keep 0: an INT8 head too; keep 3: every
+    third matrix fp16 beside INT8 ones."""
+    if backend == "int8":
+        model.quantize(None if keep is None else [int(keep and i % keep == 0) for i in range(49)])
+    odd = pkg.Dev(2 * E + 32)
+    general = pkg.GPT2WeightsGPU()
+    C.memmove(C.byref(general), C.byref(model.gpu), C.sizeof(general))
+    assert L.gpt2_d2d(odd.ptr + 2, model.gpu.layers[7].ln1_g, 2 * E) == 0
+    general.layers[7].ln1_g = odd.ptr + 2
+    scr, kv = pkg.Scratch(1), pkg.KVCache(MAXT)
+    try:
+        for pos in (0, 1, 4, 5, 31, 33, 127, 129, 255, 512, 1000, 1023):
+            token = (pos * 7919 + 3) % V
+            random_cache(pkg, L, kv, pos, pos)
+            got = step(pkg, L, model.gpu, kv, scr, backend, token, pos)
+            random_cache(pkg, L, kv, pos, pos)
+            ref = step(pkg, L, general, kv, scr, backend, token, pos)
+            assert rel_err(got[0], ref[0]) <= 1e-2, pos
+            p = np.exp(ref[0].astype(np.float64) - ref[0].max())
+            q = np.exp(got[0].astype(np.float64) - got[0].max())
+            assert float((p / p.sum() * (np.log(p / p.sum()) - np.log(q / q.sum()))).sum()) < 2e-3, pos
+            assert np.array_equal(got[1][13], ref[1][13]), pos   # the embedding
+            assert rel_err(got[1][:13], ref[1][:13]) <= 1e-2, pos
+            same = np.ones(MAXT, bool)
+            same[pos] = False
+            assert np.array_equal(got[2][:, :, :, same], ref[2][:, :, :, same]), pos   # no other row touched
+            assert rel_err(oracle.f16_to_f32(got[2][:, :, :, pos]), oracle.f16_to_f32(ref[2][:, :, :, pos])) <= 1e-2, pos
+    finally:
+        scr.free()
+        kv.free()
+        if backend == "int8":
+            L.gpt2_quant_free(C.byref(model.q))
+            model.q = None
+            model.gpu.q = None
+
+
+def test_attn_decode_edges(pkg, L):
+    """Lengths around the 8-key slots, 64-key passes and 16 waves, NaN past the length, peaked scores: against
+    float64 attention on the same fp16 values.  Probabilities and sums are fp32, so the error is the fp16
+    rounding of the output (half an ulp, 2^-11 of the value) and fp32 noise below it."""
+    rng = np.random.default_rng(5)
+    kv = pkg.KVCache(MAXT)
+    try:
+        k, v = (rng.standard_normal((H, MAXT, D), dtype=np.float32).astype(np.float16) for _ in range(2))
+        q = (4.0 * rng.standard_normal((3 * E,), dtype=np.float32)).astype(np.float16)
+        dq, out = pkg.Dev.from_numpy(q), pkg.Dev(2 * E)
+        for n in (1, 2, 7, 8, 9, 63, 64, 65, 127, 128, 129, 500, 512, 777, 1023, 1024):
+            c = np.full((12, 2, H, MAXT, D), np.float16(np.nan))
+            c[3, 0, :, :n], c[3, 1, :, :n] = k[:, :n], v[:, :n]
+            assert L.gpt2_h2d(kv.kv.data, c.ctypes.data, c.nbytes) == 0
+            L.gpt2_attn_decode(out.ptr, dq.ptr, C.byref(kv.kv), 3, n)
+            L.gpt2_sync()
+            pkg.check("attn_decode")
+            got = out.numpy(np.float16, (H, D)).astype(np.float64)
+            s = np.einsum("hjd,hd->hj", k[:, :n].astype(np.float64), q[:E].reshape(H, D).astype(np.float64)) / 8.0
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            ref = np.einsum("hj,hjd->hd", p / p.sum(axis=1, keepdims=True), v[:, :n].astype(np.float64))
+            assert np.abs(got - ref).max() <= 2.0 ** -11 * np.abs(ref).max() + 1e-5 * np.abs(v[:, :n]).max(), n
+    finally:
+        kv.free()
