@@ -1,6 +1,6 @@
 // attn_prefill.h -- causal prefill attention on the MFMA units (gfx950): one block of 16 queries
-// of one head, as a device function shared by the attention launch (attn_prefill.hip) and the
-// persistent prefill (prefill.hip).
+// of one head, as the persistent prefill (prefill.hip) runs it between its tiles; and the pieces it shares
+// with the attention launch (attn_prefill.hip), which brings keys and values in through LDS.
 //
 // Semantics of cpu/forward_cpu.c:83-116 (the reference's fused attention, cuda/kernels_fused.cu:58-140):
 // att[i, h*64 + d] = sum_{j<=i} softmax_j(q_i . k_j / 8) v_j[d] over qkv[T, 3*768] (q | k | v, head h
@@ -66,10 +66,9 @@ struct AttnLds {
 };
 
 // Queries q0 .. q0+15 of head h over keys [0, last query]; 256 threads.  Kc, Vc (optional): the
-// layer's K and V cache planes ([H][maxT][D]), filled with this block's 16 rows.  COHERENT: the
-// output rows are stored with device-scope (sc1) stores, for a consumer in the same launch on
-// another XCD.  Ends with every wave past the LDS merge (the caller may reuse `lds` after a barrier).
-template <bool COHERENT>
+// layer's K and V cache planes ([H][maxT][D]), filled with this block's 16 rows.  The output rows are stored
+// with device-scope (sc1) stores, for a consumer in the same launch on another XCD.  Ends with every wave
+// past the LDS merge (the caller may reuse `lds` after a barrier).
 __device__ __forceinline__ void attn_block(AttnLds &lds, uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
                                            int T, uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc, int maxT,
                                            int h, int q0) {
@@ -217,11 +216,8 @@ __device__ __forceinline__ void attn_block(AttnLds &lds, uint16_t *__restrict__ 
         const uint2 pk = {(uint32_t)f2h(acc[0] * inv) | ((uint32_t)f2h(acc[1] * inv) << 16),
                           (uint32_t)f2h(acc[2] * inv) | ((uint32_t)f2h(acc[3] * inv) << 16)};
         uint2 *dst = reinterpret_cast<uint2 *>(att + (size_t)q * E + h * D + 16 * wave + 4 * g);
-        if constexpr (COHERENT)
-            __hip_atomic_store(reinterpret_cast<uint64_t *>(dst), __builtin_bit_cast(uint64_t, pk), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        else
-            *dst = pk;
+        __hip_atomic_store(reinterpret_cast<uint64_t *>(dst), __builtin_bit_cast(uint64_t, pk), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 

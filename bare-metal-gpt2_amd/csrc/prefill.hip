@@ -392,7 +392,7 @@ __global__ __launch_bounds__(PF_T) void k_prefill_persist(const PFArgs a) {
                 return true;
             });
             if (ok) {
-                attn_block<true>(*reinterpret_cast<AttnLds *>(lds), ly.att, ly.qkv, T, ly.kc, ly.vc, a.maxT, h, q0);
+                attn_block(*reinterpret_cast<AttnLds *>(lds), ly.att, ly.qkv, T, ly.kc, ly.vc, a.maxT, h, q0);
                 pf_signal(cnt + cidx(l, ST_ATT, q0 / PF_RB), wave0, tr);
             }
         } else {
