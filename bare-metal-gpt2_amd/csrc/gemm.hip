@@ -922,10 +922,10 @@ static const GemmCfg kCfgs[] = {
     G2_DCFG(48, 32, 1, 2, 4),       // 10: 2 waves, wave tile 48x16
     G2_DCFG(48, 32, 3, 2, 6),       // 11: 6 waves, wave tile 16x16, 6 stages
     G2_DCFGK(32, 64, 1, 4, 4, 2),   // 12: two k groups of 4 waves (K=3072: 24 k-tiles each)
-    G2_DCFGK(32, 32, 1, 2, 4, 2),   // 13: two k groups of 2 waves
+    G2_DCFGUF(32, 32, 1, 2, 4, 2, 1), // 13: two k groups of 2 waves
     G2_DCFGK(32, 32, 1, 2, 4, 4),   // 14: four k groups of 2 waves
     G2_DCFGK(48, 32, 3, 2, 4, 2),   // 15: two k groups of 6 waves
-    G2_DCFGK(32, 64, 1, 4, 4, 3),   // 16: three k groups of 4 waves
+    G2_DCFGUF(32, 64, 1, 4, 4, 3, 1), // 16: three k groups of 4 waves
     G2_DCFGK(64, 32, 2, 2, 4, 2),   // 17: two k groups of 4 waves
     G2_DCFGK(32, 64, 1, 4, 3, 2),   // 18: two k groups of 4 waves, 3 stages
     G2_DCFG(96, 32, 3, 2, 4),       // 19: 6 waves, wave tile 32x16
@@ -946,7 +946,7 @@ static const GemmCfg kCfgs[] = {
     G2_DCFGUF(48, 64, 3, 2, 4, 1, 2),   // 34: 6 waves, wave tile 16x32 (each widened INT8 fragment feeds 2 MFMAs)
     G2_DCFGUF(48, 32, 3, 1, 4, 1, 2),   // 35: 3 waves, wave tile 16x32 (INT8 QKV, fc)
     G2_DCFGUF(48, 64, 3, 2, 4, 2, 2),   // 36: two k groups of 6 waves, wave tile 16x32
-    G2_DCFGU(96, 64, 3, 2, 4, 1, 2),    // 37: 6 waves, wave tile 32x32
+    G2_DCFGUF(96, 64, 3, 2, 4, 1, 2),   // 37: 6 waves, wave tile 32x32
     G2_DCFGUF(48, 32, 3, 1, 8, 2, 4),   // 38: two k groups of 3 waves, 8 stages, 4 k-tiles per barrier
     G2_DCFGUF(48, 32, 3, 1, 6, 2, 2),   // 39: two k groups of 3 waves, 6 stages
     G2_DCFGUF(48, 32, 3, 1, 8, 1, 4),   // 40: 3 waves, 8 stages, 4 k-tiles per barrier
@@ -966,9 +966,17 @@ static const GemmCfg kCfgs[] = {
     G2_SKCFG(96, 64, 6, 2, 4, 2, 2),    // 49: 12 waves, wave tile 16x32, 2 splits
     G2_SKCFG(96, 64, 6, 2, 4, 2, 4),    // 50: as 49, 4 splits
     G2_SKCFG(64, 64, 2, 2, 4, 2, 2),    // 51: 4 waves, wave tile 32x32, 2 splits
+    // tiles that give the trunk shapes about one work-group per CU between 257 and 1024 rows
+    G2_DCFGUF(48, 64, 3, 2, 5, 2, 1),   // 52: two k groups of 6 waves, 16x32 wave tiles, 5 stages (fp16 mlp-proj)
+    G2_DCFGUF(48, 64, 3, 1, 2, 4, 1),   // 53: four k groups of 3 waves, 16x64 wave tiles (INT8 mlp-proj)
+    G2_DCFGUF(64, 64, 2, 2, 4, 2, 2),   // 54: two k groups of 4 waves, 32x32 wave tiles (INT8 QKV, fc)
+    G2_DCFGUF(128, 64, 4, 2, 4, 1, 2),  // 55: 8 waves, wave tile 32x32, two k-tiles per barrier (INT8 QKV, fc)
+    G2_DCFGUF(144, 64, 3, 4, 4, 1, 2),  // 56: 12 waves, wave tile 48x16 (fp16 QKV, fc)
+    G2_DCFGUF(144, 64, 3, 2, 3, 2, 1),  // 57: two k groups of 6 waves, 48x32 wave tiles (INT8 QKV, fc)
+    G2_DCFGUF(96, 128, 2, 4, 4, 1, 2),  // 58: 8 waves, wave tile 48x32 (fc)
 };
 static const int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
-static_assert(sizeof(kCfgs) / sizeof(kCfgs[0]) == 52, "the pick table names configs by index");
+static_assert(sizeof(kCfgs) / sizeof(kCfgs[0]) == 59, "the pick table names configs by index");
 
 // Any K % 8 == 0 (int8: K % 16 == 0): predicated loads, one k-tile of prefetch.
 #define G2_GCFG(BN, BM, WN, WM) \
@@ -1001,8 +1009,8 @@ static const int kNumLnCfgs = (int)(sizeof(kLnCfgs) / sizeof(kLnCfgs[0]));
 
 // The LayerNorm fold's kernels, on the configs the pick table gives each role: the residual GEMMs
 // (attn-proj, mlp-proj: EPI_RESID_LN) and the GEMMs after a LayerNorm (QKV: EPI_LNF, fc:
-// EPI_LNF_GELU), fp16 and INT8 weights, every M bucket.  A call whose picked config has no entry
-// here (a forced config) runs the LayerNorm launch and the plain GEMM instead.
+// EPI_LNF_GELU), fp16 and INT8 weights, every M range.  A call whose picked config has no entry here (a
+// forced config) runs the LayerNorm launch and the plain GEMM instead.
 typedef void (*GemmLnfFn)(uint16_t *, const uint16_t *, const void *, const float *, const uint16_t *, int, int, int,
                           int, int, int, const uint16_t *, LnFold);
 struct GemmLnfEntry {
@@ -1013,36 +1021,53 @@ struct GemmLnfEntry {
 };
 #define G2_LNF(CFG, QW, EPI, BN, BM, WN, WM, S, KS, U) {CFG, QW, EPI, k_gemm_dl_lnf<BN, BM, WN, WM, S, QW, KS, U, EPI>}
 static const GemmLnfEntry kLnfKernels[] = {
-    // residual GEMMs: fp16 attn-proj 8, 25, 36 / mlp-proj 47, 23, 5; INT8 attn-proj 47, 31, 36 / mlp-proj 45, 36
-    G2_LNF(5, false, EPI_RESID_LN, 64, 64, 2, 4, 4, 1, 1),
-    G2_LNF(8, false, EPI_RESID_LN, 32, 32, 1, 2, 4, 1, 1),
-    G2_LNF(23, false, EPI_RESID_LN, 48, 32, 3, 2, 6, 2, 2),
-    G2_LNF(25, false, EPI_RESID_LN, 48, 32, 3, 2, 6, 1, 2),
+    // residual GEMMs (attn-proj, mlp-proj): fp16, then INT8
+    G2_LNF(31, false, EPI_RESID_LN, 48, 32, 3, 2, 8, 1, 4),
     G2_LNF(36, false, EPI_RESID_LN, 48, 64, 3, 2, 4, 2, 2),
     G2_LNF(47, false, EPI_RESID_LN, 32, 32, 1, 2, 4, 4, 1),
+    G2_LNF(23, false, EPI_RESID_LN, 48, 32, 3, 2, 6, 2, 2),
+    G2_LNF(16, false, EPI_RESID_LN, 32, 64, 1, 4, 4, 3, 1),
+    G2_LNF(52, false, EPI_RESID_LN, 48, 64, 3, 2, 5, 2, 1),
+    G2_LNF(47, true, EPI_RESID_LN, 32, 32, 1, 2, 4, 4, 1),
     G2_LNF(31, true, EPI_RESID_LN, 48, 32, 3, 2, 8, 1, 4),
     G2_LNF(36, true, EPI_RESID_LN, 48, 64, 3, 2, 4, 2, 2),
     G2_LNF(45, true, EPI_RESID_LN, 48, 32, 3, 1, 4, 4, 2),
-    G2_LNF(47, true, EPI_RESID_LN, 32, 32, 1, 2, 4, 4, 1),
-    // QKV: fp16 8, 29, 35, 0; INT8 47, 39, 36, 35
-    G2_LNF(0, false, EPI_LNF, 96, 64, 2, 4, 4, 1, 1),
-    G2_LNF(8, false, EPI_LNF, 32, 32, 1, 2, 4, 1, 1),
-    G2_LNF(29, false, EPI_LNF, 48, 64, 3, 4, 6, 1, 3),
+    G2_LNF(53, true, EPI_RESID_LN, 48, 64, 3, 1, 2, 4, 1),
+    // QKV: fp16, then INT8
+    G2_LNF(13, false, EPI_LNF, 32, 32, 1, 2, 4, 2, 1),
+    G2_LNF(31, false, EPI_LNF, 48, 32, 3, 2, 8, 1, 4),
+    G2_LNF(3, false, EPI_LNF, 64, 32, 2, 2, 4, 1, 1),
+    G2_LNF(32, false, EPI_LNF, 48, 64, 3, 4, 8, 1, 4),
+    G2_LNF(5, false, EPI_LNF, 64, 64, 2, 4, 4, 1, 1),
     G2_LNF(35, false, EPI_LNF, 48, 32, 3, 1, 4, 1, 2),
-    G2_LNF(35, true, EPI_LNF, 48, 32, 3, 1, 4, 1, 2),
-    G2_LNF(36, true, EPI_LNF, 48, 64, 3, 2, 4, 2, 2),
-    G2_LNF(39, true, EPI_LNF, 48, 32, 3, 1, 6, 2, 2),
+    G2_LNF(26, false, EPI_LNF, 48, 64, 3, 4, 4, 1, 2),
+    G2_LNF(1, false, EPI_LNF, 128, 64, 4, 2, 3, 1, 1),
+    G2_LNF(56, false, EPI_LNF, 144, 64, 3, 4, 4, 1, 2),
     G2_LNF(47, true, EPI_LNF, 32, 32, 1, 2, 4, 4, 1),
-    // fc: fp16 8, 40, 26, 6; INT8 47, 39, 36, 35, 1
-    G2_LNF(6, false, EPI_LNF_GELU, 128, 128, 2, 4, 4, 1, 1),
-    G2_LNF(8, false, EPI_LNF_GELU, 32, 32, 1, 2, 4, 1, 1),
-    G2_LNF(26, false, EPI_LNF_GELU, 48, 64, 3, 4, 4, 1, 2),
+    G2_LNF(39, true, EPI_LNF, 48, 32, 3, 1, 6, 2, 2),
+    G2_LNF(36, true, EPI_LNF, 48, 64, 3, 2, 4, 2, 2),
+    G2_LNF(54, true, EPI_LNF, 64, 64, 2, 2, 4, 2, 2),
+    G2_LNF(35, true, EPI_LNF, 48, 32, 3, 1, 4, 1, 2),
+    G2_LNF(55, true, EPI_LNF, 128, 64, 4, 2, 4, 1, 2),
+    G2_LNF(57, true, EPI_LNF, 144, 64, 3, 2, 3, 2, 1),
+    // fc: fp16, then INT8
+    G2_LNF(13, false, EPI_LNF_GELU, 32, 32, 1, 2, 4, 2, 1),
+    G2_LNF(31, false, EPI_LNF_GELU, 48, 32, 3, 2, 8, 1, 4),
     G2_LNF(40, false, EPI_LNF_GELU, 48, 32, 3, 1, 8, 1, 4),
-    G2_LNF(1, true, EPI_LNF_GELU, 128, 64, 4, 2, 3, 1, 1),
-    G2_LNF(35, true, EPI_LNF_GELU, 48, 32, 3, 1, 4, 1, 2),
-    G2_LNF(36, true, EPI_LNF_GELU, 48, 64, 3, 2, 4, 2, 2),
-    G2_LNF(39, true, EPI_LNF_GELU, 48, 32, 3, 1, 6, 2, 2),
+    G2_LNF(5, false, EPI_LNF_GELU, 64, 64, 2, 4, 4, 1, 1),
+    G2_LNF(26, false, EPI_LNF_GELU, 48, 64, 3, 4, 4, 1, 2),
+    G2_LNF(37, false, EPI_LNF_GELU, 96, 64, 3, 2, 4, 1, 2),
+    G2_LNF(1, false, EPI_LNF_GELU, 128, 64, 4, 2, 3, 1, 1),
+    G2_LNF(56, false, EPI_LNF_GELU, 144, 64, 3, 4, 4, 1, 2),
+    G2_LNF(58, false, EPI_LNF_GELU, 96, 128, 2, 4, 4, 1, 2),
     G2_LNF(47, true, EPI_LNF_GELU, 32, 32, 1, 2, 4, 4, 1),
+    G2_LNF(39, true, EPI_LNF_GELU, 48, 32, 3, 1, 6, 2, 2),
+    G2_LNF(36, true, EPI_LNF_GELU, 48, 64, 3, 2, 4, 2, 2),
+    G2_LNF(54, true, EPI_LNF_GELU, 64, 64, 2, 2, 4, 2, 2),
+    G2_LNF(35, true, EPI_LNF_GELU, 48, 32, 3, 1, 4, 1, 2),
+    G2_LNF(55, true, EPI_LNF_GELU, 128, 64, 4, 2, 4, 1, 2),
+    G2_LNF(57, true, EPI_LNF_GELU, 144, 64, 3, 2, 3, 2, 1),
+    G2_LNF(58, true, EPI_LNF_GELU, 96, 128, 2, 4, 4, 1, 2),
 };
 
 static int g_force_cfg = -2;  // -2: not read yet; -1: table
@@ -1067,26 +1092,40 @@ static int forced_cfg() {
     return g_force_cfg;
 }
 
-// Measured picks for the GPT-2 trunk shapes, by prompt length: each shape's 12 layer GEMMs
-// (distinct weights) back to back on MI355X, every config of the table timed per M bucket (fp16 and
-// INT8 weights), then for M in (256, 512] the whole step (12 layers x {QKV, attn-proj, fc, mlp-proj})
-// timed over per-shape candidates, because a kernel's best config alone and inside the step differ
-// (attn-proj most).  Buckets: M <= 64, <= 128, <= 256, <= 512, <= 1024; shapes QKV, attn-proj, fc,
-// mlp-proj; {fp16, INT8}.  Every config the prefill picks for attn-proj, fc and mlp-proj carries the
-// fused-epilogue kernels (gelu, residual).
-//   * short prompts take small tiles with k groups: 32x32 tiles with four k groups (47) keep 256+
-//     waves busy on mlp-proj's K=3072 (M=128: 6.6 us against 10.1 with one group) and on every INT8
-//     shape up to M=256 (M=64 QKV: 3.95 against 6.3 us), where each wave widens fewer W rows;
-//   * M in (256, 512] (the P=512 headline): 48-row W tiles, chosen inside the step;
-//   * M up to 1024: 96x64 / 128x128 tiles for fp16 QKV and fc (10.4 / 10.9 us), 64x64 for mlp-proj
-//     (12.9 against 16.5 us), 48x64 with two k groups (36) for attn-proj and the INT8 GEMMs, 128x64
-//     for INT8 fc (12.0 against 13.4 us for 48x32, isolated).
-static const int kPick[5][4][2] = {
-    /* M <= 64   */ {{8, 47}, {8, 47}, {8, 47}, {47, 47}},
-    /* M <= 128  */ {{8, 39}, {8, 47}, {8, 39}, {47, 47}},
-    /* M <= 256  */ {{29, 36}, {8, 47}, {40, 36}, {47, 45}},
-    /* M <= 512  */ {{35, 35}, {25, 31}, {26, 35}, {23, 45}},
-    /* M <= 1024 */ {{0, 35}, {36, 36}, {6, 1}, {5, 36}},
+// Measured picks for the GPT-2 trunk shapes, by prompt length: each shape's 12 layer GEMMs (distinct
+// weights) back to back on MI355X, every config of the table at 20 lengths from 33 to 1000, fp16 and INT8
+// weights.  Shapes QKV, attn-proj, fc, mlp-proj; {fp16, INT8}.  Every config that the prefill picks for
+// attn-proj, fc and mlp-proj carries the fused-epilogue kernels (gelu, residual).
+// What decides is the number of work-groups: a launch takes about as long for 130 tiles as for 256 (one per
+// CU) and half again as long for 270, so the limits below lie where a tile's count passes 256, and the
+// largest tile (fewest L2 bytes per FLOP) that still gives most CUs one wins; k groups keep its waves busy.
+// us per launch, the pick of five ranges (<= 64, 128, 256, 512, 1024) that this table replaced -> this one:
+//   fp16  QKV M=64 4.5 -> 3.9, 160 5.1 -> 4.3, 448 6.2 -> 5.7, 800 9.2 -> 7.5, 1000 10.2 -> 8.7
+//         attn-proj M=64 4.3 -> 3.7, 256 4.5 -> 4.1, 512 4.5 -> 4.2
+//         fc M=64 4.5 -> 4.0, 128 5.2 -> 4.4, 320 7.1 -> 5.9, 512 7.7 -> 7.2, 640 10.7 -> 7.6, 1000 10.9 -> 9.7
+//         mlp-proj M=320 8.3 -> 7.1, 640 13.1 -> 9.1, 1000 13.2 -> 11.5
+//   INT8  QKV M=160 5.2 -> 4.6, 448 6.6 -> 6.1, 896 10.5 -> 8.2, 1000 10.6 -> 9.7
+//         attn-proj M=320 4.4 -> 4.2
+//         fc M=320 6.5 -> 6.0, 640 9.0 -> 8.2, 1000 12.5 -> 11.1
+//         mlp-proj M=256 8.3 -> 7.9, 1000 12.3 -> 11.5
+struct PickRow {
+    int m;            // up to this M
+    int cfg[4][2];
+};
+static const PickRow kPick[] = {
+    {64, {{13, 47}, {31, 47}, {13, 47}, {47, 47}}},
+    {96, {{31, 47}, {31, 47}, {31, 39}, {47, 47}}},
+    {128, {{31, 39}, {31, 47}, {31, 39}, {47, 47}}},
+    {160, {{31, 39}, {31, 47}, {40, 36}, {47, 47}}},
+    {224, {{3, 36}, {31, 47}, {40, 36}, {47, 47}}},
+    {256, {{32, 36}, {31, 47}, {40, 36}, {47, 47}}},
+    {320, {{32, 36}, {31, 47}, {5, 54}, {47, 47}}},
+    {448, {{5, 54}, {31, 31}, {26, 35}, {23, 45}}},
+    {512, {{35, 35}, {31, 31}, {37, 35}, {23, 45}}},
+    {640, {{26, 35}, {36, 36}, {1, 55}, {16, 53}}},
+    {704, {{1, 55}, {36, 36}, {56, 57}, {52, 53}}},
+    {896, {{1, 55}, {36, 36}, {58, 58}, {52, 53}}},
+    {1024, {{56, 57}, {36, 36}, {58, 58}, {52, 53}}},
 };
 
 static int pick_cfg(int M, int N, int K, bool qw = false) {
@@ -1096,11 +1135,13 @@ static int pick_cfg(int M, int N, int K, bool qw = false) {
     else if (N == 768 && K == 768) shape = 1;        // attn-proj
     else if (N == 3072 && K == 768) shape = 2;       // fc
     else if (N == 768 && K == 3072) shape = 3;       // mlp-proj
-    if (shape >= 0 && M >= 2 && M <= 1024) {
-        const int bucket = M <= 64 ? 0 : M <= 128 ? 1 : M <= 256 ? 2 : M <= 512 ? 3 : 4;
-        const int c = kPick[bucket][shape][qw ? 1 : 0];
-        if (cfg_usable(c, M, N, K)) return c;
-    }
+    if (shape >= 0 && M >= 2)
+        for (const PickRow &r : kPick) {
+            if (M > r.m) continue;
+            const int c = r.cfg[shape][qw ? 1 : 0];
+            if (cfg_usable(c, M, N, K)) return c;
+            break;
+        }
     // Other shapes: vocabulary-sized N (the tied head, 50257 rows of W) has many tiles per CU, where
     // large tiles win on L2 bytes per FLOP (M=512: 128x64 83 us, 256x128 88, 128x128 94, 48-row
     // tiles >= 135) and the 128x64 tile double-buffered (three work-groups per CU) beats its 3-stage
