@@ -98,6 +98,7 @@ __device__ __forceinline__ void attn_tiles(uint16_t *__restrict__ att, const uin
     for (int c = wave; c < nc; c += AF_W) {
         if (c + AF_W < nc) wait_vm<8>();
         else wait_vm<0>();
+        asm volatile("" ::: "memory");
         const char *kt = ring + stage * 2 * AF_TILE, *vt = kt + AF_TILE;
         // ---- scores of keys 32 c + 16 t + 4 g + r for query q0 + 16 qt + jq
         f32x4 s[QT][2];

@@ -8,17 +8,24 @@
 // trips where one suffices.  Here:
 //   * A work-group owns 16 rows of W (one MFMA row block) and 16 rows of A; its four waves split K.
 //     Grid = (N / 16) x ceil(M / 16): 48-192 work-groups per 16 rows of A.
-//   * Each lane loads its share of its W row straight into registers (16-byte loads, all issued at
-//     once: one memory round trip), while the 16 rows of A go to LDS by direct-to-LDS loads (or, with
-//     the LayerNorm prologue, are normalized in registers and written there).
-//   * One wait, one barrier, then the wave's MFMAs (W as the A operand, the A rows as B), the four
-//     waves' sums added in LDS in wave order, and wave 0's epilogue: scale (INT8), bias, then the
-//     elementwise op as the unfused sequence would apply it (epi_out).
+//   * A wave brings its quarter of the rows of W and of A to LDS with direct loads of whole 128-byte pieces
+//     of a row (64 bytes of int8 codes), all issued at once (one memory round trip; K = 3072 fp16: W
+//     through a ring of six k-tiles, refilled as they are consumed), and multiplies each 64-wide k-tile as
+//     it lands.  Loaded as fragments straight from memory, neighbouring lanes were rows apart and an
+//     instruction took the address unit four times as long.  us per launch, fragments -> LDS: mlp-proj
+//     fp16 M = 16 5.7 -> 3.7 (host-bound now), traced in the prefill 7.0 -> 5.2; INT8 M = 48 4.8 -> 4.1;
+//     the whole prefill fp16 T = 17 330 -> 297, INT8 319 -> 304.
+//   * What a wave multiplies it loaded itself, so nothing but its own loads is waited for (with the
+//     LayerNorm prologue, A is normalized in registers, written to LDS and published by a barrier).  The
+//     four waves' sums are added in LDS in wave order; wave 0 runs the epilogue: scale (INT8), bias,
+//     then the elementwise op as the unfused sequence would apply it (epi_out).
 //   * The LayerNorm prologue (QKV after LN1, fc after LN2) normalizes the block's 16 rows with the
 //     LayerNorm kernel's arithmetic (ln_rows768: ln_row768's operations row by row, the rows'
 //     reductions interleaved), so the result is bit-identical to the LayerNorm launch followed by
 //     this kernel.  Its rows are loaded before the weights and normalized while the weight stream
 //     is in flight.
+#include <type_traits>
+
 #include "common.h"
 
 namespace g2 {
@@ -27,46 +34,45 @@ constexpr int SKN_W = 4;      // waves per work-group: K split four ways
 constexpr int SKN_MB = 16;    // rows of A per work-group (the MFMA's B columns)
 [[maybe_unused]] constexpr int SKN_TILE = SKN_MB * 128;   // LDS bytes per 64-wide k-tile of the A block
 
-// k offset, inside a wave's share of K, of the 8 values lane group g feeds to MFMA step s.  INT8
-// pairs steps 2t and 2t+1 so that one 16-byte load holds both of a lane's slots (k = 64t + 16g + 8h);
-// fp16 takes k = 32s + 8g.  A and W use the same map, so every k meets its partner once.
-template <bool QW>
-__device__ __forceinline__ int skn_k(int s, int g) {
-    return QW ? 64 * (s >> 1) + 16 * g + 8 * (s & 1) : 32 * s + 8 * g;
+// f(t) for t = T0 .. T1 - 1, t a compile-time constant.
+template <int T0, int T1, class F>
+__device__ __forceinline__ void unroll_tiles(F f) {
+    if constexpr (T0 < T1) {
+        f(std::integral_constant<int, T0>{});
+        unroll_tiles<T0 + 1, T1>(f);
+    }
 }
 
 template <int K, bool QW, int EPI, bool LNP>
-__global__ __launch_bounds__(64 * SKN_W) void k_gemm_skinny(uint16_t *__restrict__ C, const uint16_t *__restrict__ A,
-                                                            const void *__restrict__ Wv, const float *__restrict__ Ws,
-                                                            const uint16_t *__restrict__ bias, int M, int N, int nbn,
-                                                            const uint16_t *resid, const uint16_t *__restrict__ ln_g,
-                                                            const uint16_t *__restrict__ ln_b) {
+__device__ __forceinline__ void gemm_skinny_wg(uint16_t *__restrict__ C, const uint16_t *__restrict__ A,
+                                               const void *__restrict__ Wv, const float *__restrict__ Ws,
+                                               const uint16_t *__restrict__ bias, int M, int N, int nbn,
+                                               const uint16_t *resid, const uint16_t *__restrict__ ln_g,
+                                               const uint16_t *__restrict__ ln_b) {
 #if defined(__HIP_DEVICE_COMPILE__)   // LDS address-space pointers exist only in the device pass
     constexpr int KT = K / 64;              // 64-wide k-tiles of the A block
-    constexpr int KW = K / SKN_W;           // one wave's share of K
-    constexpr int NS = KW / 32;             // MFMA steps per wave
-    constexpr int NL = QW ? NS / 2 : NS;    // 16-byte W loads per lane
-    static_assert(KW % 64 == 0, "a wave's share of K is whole 64-wide tiles");
+    constexpr int WT = KT / SKN_W;          // a wave's share of them
+    constexpr int WTILE = QW ? 1024 : 2048; // LDS bytes of a k-tile of the W block
+    constexpr int WR = (QW || WT <= 6) ? WT : 6;   // W k-tiles in a wave's ring (fp16 K = 3072: all do not fit)
+    constexpr int WI = WTILE / 1024, AI = 2;   // load instructions per k-tile: W, A
+    static_assert(KT % SKN_W == 0, "a wave's share of K is whole 64-wide tiles");
     static_assert(!LNP || (K == GPT2_N_EMBD && EPI != EPI_RESID), "the LayerNorm prologue: K = 768, no residual");
-    static_assert((2 * KT) % SKN_W == 0, "the A block's loads split evenly over the waves");
-    // A block [KT][16 rows][128 B] (16-byte chunk c of row r at slot c ^ (r & 7)), then the sums of
-    // waves 1..3
-    __shared__ __attribute__((aligned(1024))) char lds[KT * SKN_TILE + (SKN_W - 1) * 64 * 16];
-    char *const xs = lds;
-    f32x4 *const red = reinterpret_cast<f32x4 *>(lds + KT * SKN_TILE);
+    static_assert(WT * (AI + WI) < 64, "a wave's loads are counted");
+    // A block [KT][16 rows][128 B] and the waves' W rings [WR][16 rows][128 or 64 B] (16-byte chunk c of row r
+    // at slot c ^ (r & 7), or c ^ (r / 4 & 3)), then the sums of waves 1..3.  One LDS object: with several, the
+    // compiler waits for every direct load in flight ahead of the first fragment read.
+    __shared__ __attribute__((aligned(1024))) char lds[KT * SKN_TILE + SKN_W * WR * WTILE + (SKN_W - 1) * 64 * 16];
+    f32x4 *const red = reinterpret_cast<f32x4 *>(lds + KT * SKN_TILE + SKN_W * WR * WTILE);
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lrow = lane & 15, g = lane >> 4;
     const int nb = blockIdx.x % nbn, mb = blockIdx.x / nbn;
     const int n0 = nb * 16, m0 = mb * SKN_MB;
-    const int kw0 = wave * KW;
+    char *const xs = lds + wave * WT * SKN_TILE;                         // this wave's A tiles
+    char *const ws = lds + KT * SKN_TILE + wave * WR * WTILE;            // and W ring
 
-    // Loads, in this order (loads complete in issue order, so a wait for one is a wait for every
-    // load issued before it): the LayerNorm prologue's rows and gamma / beta (L2-resident, needed
-    // first), this lane's share of W row n0 + lrow (N % 16 == 0: the row exists; all of it in flight
-    // at once, from HBM the longest wait), then the epilogue operands.  Compiler barriers keep the
-    // order (left to itself the compiler moves the weight loads behind the LayerNorm and the epilogue
-    // operands behind the A block's wait).
+    // Loads, in this order (they complete in issue order): the LayerNorm prologue's rows and gamma / beta
+    // (L2-resident, needed first), the epilogue operands, then the k-tiles.  Compiler barriers keep it.
     f16x4 lg[3], lb[3], lx[4][3];   // LayerNorm prologue: rows wave + 4 r; lane l: elements 256 i + 4 l ..
     if constexpr (LNP) {
 #pragma unroll
@@ -82,15 +88,6 @@ __global__ __launch_bounds__(64 * SKN_W) void k_gemm_skinny(uint16_t *__restrict
         }
         asm volatile("" ::: "memory");
     }
-    i32x4 wl[NL];
-    {
-        const char *wrow = reinterpret_cast<const char *>(Wv) + (size_t)(n0 + lrow) * K * (QW ? 1 : 2);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int k = kw0 + (QW ? skn_k<true>(2 * i, g) : skn_k<false>(i, g));
-            wl[i] = *reinterpret_cast<const i32x4 *>(wrow + (size_t)k * (QW ? 1 : 2));
-        }
-    }
     // the lane's outputs C[m][nbase .. nbase+3]: scales, bias and residual (rows past M read row M-1
     // and store nothing; the residual may alias C: this lane alone writes those elements)
     const int nbase = n0 + 4 * g, m = m0 + lrow;
@@ -105,17 +102,52 @@ __global__ __launch_bounds__(64 * SKN_W) void k_gemm_skinny(uint16_t *__restrict
     uint2 rs = {0u, 0u};
     if constexpr (EPI == EPI_RESID) rs = *reinterpret_cast<const uint2 *>(resid + (size_t)min(m, M - 1) * N + nbase);
     asm volatile("" ::: "memory");
+    // k-tile t of this wave's share: A rows 8 q .. + 7 (lane l slot l & 7 of row 8 q + l / 8), W the same
+    // way or, int8, 16 rows of 64 bytes an instruction (lane l slot l & 3 of row l / 4); N % 16 == 0, so
+    // every row of W exists
+    const int r8 = lane >> 3, c8 = ((lane & 7) ^ r8) * 8;
+    const int r4 = lane >> 2, c4 = ((lane & 3) ^ ((r4 >> 2) & 3)) * 16;
+    auto issue_a = [&](int t) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            __builtin_amdgcn_global_load_lds(A + (size_t)min(m0 + 8 * q + r8, M - 1) * K + 64 * (wave * WT + t) + c8,
+                                             G2_LDS(xs + t * SKN_TILE + 1024 * q), 16, 0, 0);
+    };
+    auto issue_w = [&](int t) {
+        const int k0 = 64 * (wave * WT + t);
+        char *dst = ws + (t % WR) * WTILE;
+        if constexpr (QW) {
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const int8_t *>(Wv) + (size_t)(n0 + r4) * K + k0 + c4,
+                                             G2_LDS(dst), 16, 0, 0);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint16_t *>(Wv) + (size_t)(n0 + 8 * q + r8) * K + k0 + c8,
+                                                 G2_LDS(dst + 1024 * q), 16, 0, 0);
+        }
+    };
     if constexpr (LNP) {
+        // The prologue form takes W through registers, lane for lane what the direct loads would have put in
+        // LDS: with direct loads in flight the compiler counts no ordinary load exactly, and the LayerNorm
+        // would start when W has landed instead of running meanwhile.
+        i32x4 wl[WT * WI];
+#pragma unroll
+        for (int t = 0; t < WT; ++t)
+#pragma unroll
+            for (int q = 0; q < WI; ++q) {
+                const int k0 = 64 * (wave * WT + t);
+                wl[t * WI + q] = QW ? *reinterpret_cast<const i32x4 *>(reinterpret_cast<const int8_t *>(Wv) + (size_t)(n0 + r4) * K + k0 + c4)
+                                    : *reinterpret_cast<const i32x4 *>(reinterpret_cast<const uint16_t *>(Wv) +
+                                                                       (size_t)(n0 + 8 * q + r8) * K + k0 + c8);
+            }
+        asm volatile("" ::: "memory");
         // the LayerNorm's inputs pass through here, so none of its arithmetic is scheduled ahead of
         // the loads above (the compiler would otherwise issue the weight loads after it)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(lx[r][i]) : : "memory");
-    }
-
-    if constexpr (LNP) {
-        // normalized as the LayerNorm kernel does, written where the direct-to-LDS load would have put them
+        // normalized as the LayerNorm kernel does, written where a direct-to-LDS load would have put them
         f16x4 o[4][3];
         ln_rows768<4>(lx, lg, lb, o);
 #pragma unroll
@@ -123,43 +155,55 @@ __global__ __launch_bounds__(64 * SKN_W) void k_gemm_skinny(uint16_t *__restrict
             const int row = wave + 4 * r;
 #pragma unroll
             for (int i = 0; i < 3; ++i)   // element 256 i + 4 lane: k-tile 4 i + lane / 16, chunk (lane & 15) / 2
-                *reinterpret_cast<f16x4 *>(xs + (4 * i + (lane >> 4)) * SKN_TILE + row * 128 +
+                *reinterpret_cast<f16x4 *>(lds + (4 * i + (lane >> 4)) * SKN_TILE + row * 128 +
                                            ((((lane & 15) >> 1) ^ (row & 7)) << 4) + (lane & 1) * 8) = o[r][i];
         }
+        asm volatile("" ::: "memory");   // W is waited for here, not inside the LayerNorm
+#pragma unroll
+        for (int i = 0; i < WT * WI; ++i) *reinterpret_cast<i32x4 *>(ws + 1024 * i + 16 * lane) = wl[i];
+        lds_barrier();
     } else {
-        // load q (two per k-tile) fills rows 8 (q & 1) .. +7 of tile q / 2, lane l slot l & 7 of row
-        // 8 (q & 1) + l / 8; wave w issues q = w, w + 4, ...
 #pragma unroll
-        for (int j = 0; j < 2 * KT / SKN_W; ++j) {
-            const int q = wave + SKN_W * j;
-            const int r = 8 * (q & 1) + (lane >> 3), c = (lane & 7) ^ (r & 7);
-            const uint16_t *src = A + (size_t)min(m0 + r, M - 1) * K + 64 * (q >> 1) + 8 * c;
-            __builtin_amdgcn_global_load_lds(src, G2_LDS(xs + q * 1024), 16, 0, 0);
+        for (int t = 0; t < WR; ++t) {
+            issue_a(t);
+            issue_w(t);
         }
-    }
-    // the direct-to-LDS A block is complete when this wave's loads have all landed (the LayerNorm
-    // path wrote its rows with LDS stores); the barrier then publishes every wave's part
-    if constexpr (!LNP) wait_vm<0>();
-    lds_barrier();
-    // the weights are used from here on (the compiler would otherwise widen INT8 codes inside the
-    // LayerNorm prologue, waiting there for the weight stream)
 #pragma unroll
-    for (int i = 0; i < NL; ++i) asm volatile("" : "+v"(wl[i]));
+        for (int t = WR; t < WT; ++t) issue_a(t);
+    }
 
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto consume = [&](int t) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        f16x8 w;
-        if constexpr (QW) {
-            const i32x4 v = wl[s >> 1];
-            w = i8x8_to_f16x8((s & 1) ? uint2{(uint32_t)v[2], (uint32_t)v[3]} : uint2{(uint32_t)v[0], (uint32_t)v[1]});
-        } else {
-            w = __builtin_bit_cast(f16x8, wl[s]);
+        for (int s = 0; s < 2; ++s) {
+            const int c = 4 * s + g;   // 16-byte chunk of the lane's eight k
+            f16x8 w;
+            if constexpr (QW) {
+                const char *p = ws + (t % WR) * WTILE + lrow * 64 + (((c >> 1) ^ ((lrow >> 2) & 3)) << 4) + 8 * (c & 1);
+                w = i8x8_to_f16x8(*reinterpret_cast<const uint2 *>(p));
+            } else {
+                w = *reinterpret_cast<const f16x8 *>(ws + (t % WR) * WTILE + lrow * 128 + ((c ^ (lrow & 7)) << 4));
+            }
+            const f16x8 x = *reinterpret_cast<const f16x8 *>(xs + t * SKN_TILE + lrow * 128 + ((c ^ (lrow & 7)) << 4));
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0);
         }
-        const int k = kw0 + skn_k<QW>(s, g), c = (k & 63) >> 3;
-        const f16x8 x = *reinterpret_cast<const f16x8 *>(xs + (k >> 6) * SKN_TILE + lrow * 128 + ((c ^ (lrow & 7)) << 4));
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0);
-    }
+    };
+    // tile t has landed when at most the loads issued behind its last one are outstanding: the rest of the
+    // first WR tiles, the later A tiles, and the refills since
+    static_assert(WT == WR || WT == 2 * WR, "every slot of the ring is refilled once, or never");
+    unroll_tiles<0, WT>([&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        if constexpr (!LNP) {
+            wait_vm<t < WR ? (WR - 1 - t) * (AI + WI) + (WT - WR) * AI + (WT > WR ? t * WI : 0) : (WT - 1 - t) * WI>();
+            asm volatile("" ::: "memory");
+        }
+        consume(t);
+        if constexpr (t + WR < WT) {
+            // the slot's fragments have been read before the refill goes out
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(acc) : : "memory");
+            issue_w(t + WR);
+        }
+    });
     // lane holds D[n0 + 4g + i][m0 + lrow]; waves 1..3 hand theirs to wave 0, added in wave order
     if (wave > 0) red[(wave - 1) * 64 + lane] = acc;
     lds_barrier();
@@ -178,6 +222,17 @@ __global__ __launch_bounds__(64 * SKN_W) void k_gemm_skinny(uint16_t *__restrict
     *reinterpret_cast<uint2 *>(C + (size_t)m * N + nbase) =
         uint2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
 #endif
+}
+
+// The pointers reach the body as __restrict__ parameters of an inlined function, so the compiler knows that
+// its LDS reads do not alias the direct loads in flight (it would wait for them ahead of every read).
+template <int K, bool QW, int EPI, bool LNP>
+__global__ __launch_bounds__(64 * SKN_W) void k_gemm_skinny(uint16_t *__restrict__ C, const uint16_t *__restrict__ A,
+                                                            const void *__restrict__ Wv, const float *__restrict__ Ws,
+                                                            const uint16_t *__restrict__ bias, int M, int N, int nbn,
+                                                            const uint16_t *resid, const uint16_t *__restrict__ ln_g,
+                                                            const uint16_t *__restrict__ ln_b) {
+    gemm_skinny_wg<K, QW, EPI, LNP>(C, A, Wv, Ws, bias, M, N, nbn, resid, ln_g, ln_b);
 }
 
 typedef void (*SkinnyFn)(uint16_t *, const uint16_t *, const void *, const float *, const uint16_t *, int, int, int,
