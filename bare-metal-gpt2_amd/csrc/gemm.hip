@@ -675,49 +675,13 @@ __device__ __forceinline__ void gemm_dl(uint16_t *__restrict__ C, const uint16_t
             rsd_e[b] = 1.0f / sqrtf(var + GPT2_LN_EPS);
         }
     }
-    // Epilogue: lane holds D[n][m] for n = nb..nb+3, m = mrow.
-    if (!vec_store) {
-        if constexpr (RLN || LNF) return;   // the host runs the fold only where C rows are 8-byte aligned
-        else {
-        // Rows of C that are not 8-byte aligned (odd N: the tied head's 50257 columns): the tile
-        // is staged in the now idle LDS ring and leaves row by row, a wave writing 64 consecutive
-        // column pairs per store (dword-aligned in C; a lone first or last column as a 2-byte
-        // store), instead of 2-byte stores scattered over 16 rows per instruction.
-        constexpr int CS = BN + 4;   // staged row stride (halves): rows 8 bytes apart in banks
-        static_assert(BM * CS * 2 <= KS * S * STAGE, "staged C tile fits the LDS ring");
-        uint16_t *ct = reinterpret_cast<uint16_t *>(smem_all);
-        lds_barrier();   // every wave is done with the last k-tile's fragments (and the k-group sums)
-#pragma unroll
-        for (int a = 0; a < TN && kg == 0; ++a) {
-            const int nl = wn0 + a * 16 + lgrp * 4;
-#pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                const int ml = wm0 + b * 16 + lrow;
-                uint16_t o[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float v = acc[a][b][i];
-                    if constexpr (QW) v = v * sc_e[a][i];
-                    o[i] = epi_out<EPI>(v + (bias ? h2f((uint16_t)bs_e[a][i]) : 0.f), rs_at(a, b, i));
-                }
-                *reinterpret_cast<uint2 *>(ct + ml * CS + nl) =
-                    uint2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-            }
-        }
-        lds_barrier();
-        const int ncols = min(BN, N - n0);
-        for (int r = wave_all; r < BM && m0 + r < M; r += NW * KS) {
-            const uint16_t *src = ct + r * CS;
-            uint16_t *dst = C + (size_t)(m0 + r) * N + n0;
-            const int head = (int)(((uintptr_t)dst >> 1) & 1);   // column 0 is not 4-byte aligned
-            for (int c = head + 2 * lane; c + 1 < ncols; c += 128)
-                *reinterpret_cast<uint32_t *>(dst + c) = (uint32_t)src[c] | ((uint32_t)src[c + 1] << 16);
-            if (lane == 0 && head) dst[0] = src[0];
-            if (lane == 1 && ((ncols - head) & 1)) dst[ncols - 1] = src[ncols - 1];
-        }
-        return;
-        }
-    }
+    // Epilogue: lane holds D[n][m] for n = nb..nb+3, m = mrow, and stores them as one 8-byte store, whatever the
+    // alignment of C's rows (odd N, the tied head's 50257 columns, leaves three rows in four 2, 4 or 6 bytes
+    // past a multiple of 8; the hardware takes such stores).  Staging such tiles through LDS to store whole row
+    // pieces measured the same or slower (1024 x 50257, 768 inputs: 192x128 tiles 121.5 us staged, 118 direct)
+    // and barred tiles larger than the ring; even rows store faster (50256 columns: 107).
+    if constexpr (RLN || LNF)
+        if (!vec_store) return;   // the host runs the fold only where C rows are 8-byte aligned
     if (kg != 0) return;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
@@ -759,9 +723,9 @@ __device__ __forceinline__ void gemm_dl(uint16_t *__restrict__ C, const uint16_t
             }
             if (m >= M) continue;
             uint16_t *dst = C + (size_t)m * N + nb;
-            if (vec_store && nb + 3 < N) {
+            if (nb + 3 < N) {
                 const uint2 pk = {(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-                *reinterpret_cast<uint2 *>(dst) = pk;
+                __builtin_memcpy(dst, &pk, 8);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -974,9 +938,11 @@ static const GemmCfg kCfgs[] = {
     G2_DCFGUF(144, 64, 3, 4, 4, 1, 2),  // 56: 12 waves, wave tile 48x16 (fp16 QKV, fc)
     G2_DCFGUF(144, 64, 3, 2, 3, 2, 1),  // 57: two k groups of 6 waves, 48x32 wave tiles (INT8 QKV, fc)
     G2_DCFGUF(96, 128, 2, 4, 4, 1, 2),  // 58: 8 waves, wave tile 48x32 (fc)
+    G2_DCFG(192, 128, 4, 2, 2),         // 59: 8 waves, wave tile 48x64, double-buffered (vocabulary-sized N)
+    G2_DCFG(128, 128, 4, 2, 2),         // 60: 8 waves, wave tile 32x64, double-buffered (vocabulary-sized N)
 };
 static const int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
-static_assert(sizeof(kCfgs) / sizeof(kCfgs[0]) == 59, "the pick table names configs by index");
+static_assert(sizeof(kCfgs) / sizeof(kCfgs[0]) == 61, "the pick table names configs by index");
 
 // Any K % 8 == 0 (int8: K % 16 == 0): predicated loads, one k-tile of prefetch.
 #define G2_GCFG(BN, BM, WN, WM) \
@@ -1143,15 +1109,28 @@ static int pick_cfg(int M, int N, int K, bool qw = false) {
             if (cfg_usable(c, M, N, K)) return c;
             break;
         }
-    // Other shapes: vocabulary-sized N (the tied head, 50257 rows of W) has many tiles per CU, where
-    // large tiles win on L2 bytes per FLOP (M=512: 128x64 83 us, 256x128 88, 128x128 94, 48-row
-    // tiles >= 135) and the 128x64 tile double-buffered (three work-groups per CU) beats its 3-stage
-    // form (64 vs 74 us).  Few rows and a long K: four k groups per tile keep more waves busy.
+    // Other shapes.  Few rows and a long K: four k groups per tile keep more waves busy.
+    if (M <= 64 && K >= 2048 && N <= 4096 && cfg_fits(47, K)) return 47;
+    // Vocabulary-sized N (the tied head, 50257 rows of W) has many tiles per CU, and what bounds it is what each
+    // tile reads through L2 per FLOP: double-buffered tiles of 128 rows of A, unless the last of them would be
+    // half empty, where 64-row tiles do less padding.  768 inputs, us, 128x64 tile against the chosen one:
+    //   fp16  65-128 rows 128x128 (100 rows 23.9 -> 18.7), 193-256 and 321-384 too (224: 37.4 -> 35.2, 384: 52.4
+    //         -> 50.0), from 449 on 192x128 (512: 68.5 -> 62.3, 777: 112.6 -> 99.4, 1024: 150.1 -> 118.5; 128x128
+    //         63.8, 104.6, 129.1); 128x64 stays ahead at 160 rows (27.4, 128x128 over 35), 320 (42.2, 44.0) and
+    //         448 (57.4, 60.0)
+    //   INT8  128x128 (100: 24.1 -> 18.7, 320: 46.6 -> 44.0, 512: 73.4 -> 61.8, 1024: 151.4 -> 120.2; 192x128
+    //         there 137.0), 128x64 only to 64 rows (13.9, 17.5) and at 129-192 (160: 30.1, 35.2)
+    // Below one work-group per CU the small tile's count wins (16384 columns, 100 rows: 128 work-groups of 128x128
+    // 11.4 us, 256 of 128x64 8.5; from 256 on 128x128: 16384 x 256 rows 12.9 -> 12.8, INT8 13.5 -> 12.2).
+    if (N >= 16384 && M > 32) {
+        const int mt = cdiv(M, 64);   // 64-row tiles; odd: half of the last 128-row tile is padding
+        const bool half = mt % 2 == 1 && mt <= (qw ? 3 : 7);
+        int c = 46;
+        if (!half && (long)cdiv(N, 128) * cdiv(M, 128) >= 256) c = !qw && mt > 7 ? 59 : 60;
+        if (cfg_fits(c, K)) return c;
+    }
     // Otherwise the largest tile that still gives about one work-group per CU (256 CUs), among the
     // configs whose K constraint holds; -1 when none does (the guarded kernel runs).
-    if (M <= 64 && K >= 2048 && N <= 4096 && cfg_fits(47, K)) return 47;
-    if (N >= 16384 && M > 32 && cfg_fits(46, K)) return 46;
-    if (N >= 16384 && M > 32 && cfg_fits(1, K)) return 1;
     const int order[] = {6, 0, 5, 2, 3, 8};
     int last = -1;
     for (int c : order) {
