@@ -193,7 +193,7 @@ __global__ void k_add8(f16x8 *__restrict__ x, const f16x8 *__restrict__ y, size_
 // Decode attention: one work-group per head, NW waves split the keys [0, len) (attn.h's layout, 64 keys
 // a wave and pass; a cache of 1024 positions is one pass), every load of a pass issued before its first
 // use; the waves' (m, l, c) states meet in LDS.  Bound by latency: a head's 256 KB of keys and values at
-// 1000 positions come through one CU.
+// 1000 positions come through one CU: 5.9 us, 8.8 with a lane per key row (a wave's load then touched 64 rows).
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_attn_decode(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
                                                          const uint16_t *__restrict__ Kc, const uint16_t *__restrict__ Vc,
