@@ -33,10 +33,19 @@ __device__ __forceinline__ float slot_sum(float v) {
 }
 
 // LPR lanes per row, CPL 16-byte chunks per lane (row = LPR*CPL chunks), U rows per slot in flight.
-template <int LPR, int CPL, int U, bool QW>
+// LN: x is the residual stream and the kernel applies LayerNorm(x; ln_g, ln_b) to it first.  The
+//     LPR lanes of a row slot hold all K values of x between them, so the statistics need no extra
+//     loads: each lane sums its values and the slot reduces (mean, then the biased variance of
+//     x - mean, eps inside the sqrt -- the same formula as k_layernorm); the normalized value is
+//     rounded to fp16, as the standalone LayerNorm's output would be.
+// EPI: EPI_GELU applies gelu_new to (acc*s + bias); EPI_RESID writes resid[n] + (acc*s + bias)
+//     (resid may alias C: each output is read and written by the same lane).
+template <int LPR, int CPL, int U, bool QW, bool LN = false, int EPI = EPI_NONE>
 __global__ __launch_bounds__(256) void k_gemv(uint16_t *C, const uint16_t *__restrict__ x,
                                               const void *__restrict__ Wv, const float *Ws,
-                                              const uint16_t *bias, int N) {
+                                              const uint16_t *bias, int N,
+                                              const uint16_t *ln_g, const uint16_t *ln_b,
+                                              const uint16_t *resid) {
     constexpr int RPW = 64 / LPR;                  // row slots per wave
     constexpr int ROWB = LPR * CPL * 16;           // bytes per weight row
     constexpr int XV = QW ? 2 * CPL : CPL;         // f16x8 x vectors per lane
@@ -64,22 +73,55 @@ __global__ __launch_bounds__(256) void k_gemv(uint16_t *C, const uint16_t *__res
         for (int i = 0; i < CPL; ++i)
             wv[u][i] = *reinterpret_cast<const i32x4 *>(W + (size_t)r * ROWB + (j + LPR * i) * 16);
     }
-    // The rows' scale and bias are loaded with the weights,
+    // The rows' scale, bias and residual (and the LayerNorm parameters) are loaded with the weights,
     // unconditionally at clamped rows (without a bias, x[0] stands in and is not used), each value
     // in its own register until the epilogue: loaded after the reduction, they would cost a second
     // memory round trip per launch.
     float sc_e[U];
-    uint32_t bs_e[U];
+    uint32_t bs_e[U], rs_e[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int r = min(rbase + u * RPW, N - 1);
         sc_e[u] = 1.f;
         if constexpr (QW) sc_e[u] = Ws[r];
         bs_e[u] = *(bias ? bias + r : x);
+        rs_e[u] = 0u;
+        if constexpr (EPI == EPI_RESID) rs_e[u] = resid[r];
+    }
+    f16x8 lg[LN ? XV : 1], lb[LN ? XV : 1];
+    if constexpr (LN) {
+#pragma unroll
+        for (int v = 0; v < XV; ++v) {
+            lg[v] = *reinterpret_cast<const f16x8 *>(ln_g + xoff(v));
+            lb[v] = *reinterpret_cast<const f16x8 *>(ln_b + xoff(v));
+        }
     }
     // keeps the compiler from sinking those loads down to their use (no wait is implied; the
     // pointers are not __restrict__, so the loads cannot move across this point)
     asm volatile("" ::: "memory");
+
+    if constexpr (LN) {
+        constexpr float invK = 1.0f / (float)(XV * 8 * LPR);
+        float sum = 0.f;
+#pragma unroll
+        for (int v = 0; v < XV; ++v)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += (float)xr[v][e];
+        const float mean = slot_sum<LPR>(sum) * invK;
+        float sq = 0.f;
+#pragma unroll
+        for (int v = 0; v < XV; ++v)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float d = (float)xr[v][e] - mean;
+                sq += d * d;
+            }
+        const float rstd = 1.0f / sqrtf(slot_sum<LPR>(sq) * invK + GPT2_LN_EPS);
+#pragma unroll
+        for (int v = 0; v < XV; ++v)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xr[v][e] = (f16)(((float)xr[v][e] - mean) * rstd * (float)lg[v][e] + (float)lb[v][e]);
+    }
 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -95,6 +137,8 @@ __global__ __launch_bounds__(256) void k_gemv(uint16_t *C, const uint16_t *__res
         float v = acc;
         if constexpr (QW) v *= sc_e[u];
         if (bias) v += h2f((uint16_t)bs_e[u]);
+        if constexpr (EPI == EPI_GELU) v = gelu_tanh(v);
+        if constexpr (EPI == EPI_RESID) v += h2f((uint16_t)rs_e[u]);
         if (j == 0 && r < N) C[r] = f2h(v);
     }
 }
@@ -123,7 +167,8 @@ __global__ __launch_bounds__(256) void k_gemv_generic(uint16_t *__restrict__ C, 
     }
 }
 
-typedef void (*GemvFn)(uint16_t *, const uint16_t *, const void *, const float *, const uint16_t *, int);
+typedef void (*GemvFn)(uint16_t *, const uint16_t *, const void *, const float *, const uint16_t *, int,
+                       const uint16_t *, const uint16_t *, const uint16_t *);
 
 struct GemvCfg {
     int row_chunks;   // 16-byte chunks per row this kernel is built for
@@ -188,7 +233,8 @@ void gemv(uint16_t *C, const uint16_t *x, const void *W, const float *Ws, const 
         const GemvCfg &g = kGv[c];
         const int waves = cdiv(N, g.rows_per_wave);
         const int blocks = cdiv(waves, g.waves_per_block);
-        hipLaunchKernelGGL(g.fn, dim3(blocks), dim3(64 * g.waves_per_block), 0, stream(), C, x, W, Ws, bias, N);
+        hipLaunchKernelGGL(g.fn, dim3(blocks), dim3(64 * g.waves_per_block), 0, stream(), C, x, W, Ws, bias, N,
+                           nullptr, nullptr, nullptr);
         check_launch(qw ? "k_gemv<int8>" : "k_gemv<fp16>");
         return;
     }
@@ -196,6 +242,41 @@ void gemv(uint16_t *C, const uint16_t *x, const void *W, const float *Ws, const 
     if (qw) hipLaunchKernelGGL(k_gemv_generic<true>, dim3(blocks), dim3(256), 0, stream(), C, x, W, Ws, bias, N, K);
     else hipLaunchKernelGGL(k_gemv_generic<false>, dim3(blocks), dim3(256), 0, stream(), C, x, W, Ws, bias, N, K);
     check_launch("k_gemv_generic");
+}
+
+// Fused decode GEMVs: (LayerNorm ->) GEMV (-> gelu | + residual).  Returns false when no fused
+// kernel covers the shape (the caller then runs the unfused sequence).
+struct FusedGemv {
+    int row_chunks;
+    bool qw, ln;
+    int epi;
+    int rows_per_wave;
+    GemvFn fn;
+};
+
+#define G2_FG(LPR, CPL, QW, LN, EPI) {LPR * CPL, QW, LN, EPI, 64 / LPR, k_gemv<LPR, CPL, 1, QW, LN, EPI>}
+static const FusedGemv kFused[] = {
+    G2_FG(16, 3, true, true, EPI_NONE),  G2_FG(16, 3, true, true, EPI_GELU),   G2_FG(16, 3, true, false, EPI_RESID),
+    G2_FG(64, 3, true, false, EPI_RESID),
+    G2_FG(16, 6, false, true, EPI_NONE), G2_FG(16, 6, false, true, EPI_GELU),  G2_FG(16, 6, false, false, EPI_RESID),
+    G2_FG(64, 6, false, false, EPI_RESID),
+};
+
+bool gemv_fused(uint16_t *C, const uint16_t *x, const void *W, const float *Ws, const uint16_t *bias, int N, int K,
+                bool qw, const uint16_t *ln_g, const uint16_t *ln_b, int epi, const uint16_t *resid) {
+    const bool ln = ln_g != nullptr;
+    const long row_bytes = qw ? (long)K : 2L * K;
+    if (N <= 0 || K <= 0 || row_bytes % 16 || !aligned16(W) || !aligned16(x)) return false;
+    if (ln && (!aligned16(ln_g) || !aligned16(ln_b))) return false;
+    const int rc = (int)(row_bytes / 16);
+    for (const FusedGemv &f : kFused) {
+        if (f.row_chunks != rc || f.qw != qw || f.ln != ln || f.epi != epi) continue;
+        const int blocks = cdiv(cdiv(N, f.rows_per_wave), 4);
+        hipLaunchKernelGGL(f.fn, dim3(blocks), dim3(256), 0, stream(), C, x, W, Ws, bias, N, ln_g, ln_b, resid);
+        check_launch("k_gemv<fused>");
+        return true;
+    }
+    return false;
 }
 
 }  // namespace g2

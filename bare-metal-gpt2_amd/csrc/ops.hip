@@ -194,18 +194,23 @@ __global__ void k_add8(f16x8 *__restrict__ x, const f16x8 *__restrict__ y, size_
 // a wave and pass; a cache of 1024 positions is one pass), every load of a pass issued before its first
 // use; the waves' (m, l, c) states meet in LDS.  Bound by latency: a head's 256 KB of keys and values at
 // 1000 positions come through one CU: 5.9 us, 8.8 with a lane per key row (a wave's load then touched 64 rows).
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_attn_decode(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
-                                                         const uint16_t *__restrict__ Kc, const uint16_t *__restrict__ Vc,
-                                                         int maxT, StepArg st_arg, int len_imm) {
-    constexpr int D = GPT2_HEAD_DIM, NT = 8;
+// APPEND: the last key and value are the qkv row's own, which the caller is writing to the cache meanwhile.
+template <int NW, bool APPEND>
+__device__ __forceinline__ void attn_decode_wg(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
+                                               const uint16_t *__restrict__ Kc, const uint16_t *__restrict__ Vc,
+                                               int maxT, int len, int h) {
+    constexpr int E = GPT2_N_EMBD, D = GPT2_HEAD_DIM, NT = 8;
     __shared__ float sm[NW], sl[NW], sc[NW][D];
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = blockIdx.x;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = lane >> 3, dg = (lane & 7) * 8;
-    const int len = min(len_imm > 0 ? len_imm : st_arg.p() + 1, maxT);
     const int per = ((len + NW - 1) / NW + 7) & ~7;   // keys per wave (multiple of 8)
     const int j0 = min(len, w * per), j1 = min(len, j0 + per);
     const uint16_t *kb = Kc + (size_t)h * maxT * D + dg, *vb = Vc + (size_t)h * maxT * D + dg;
+    auto row = [&](const uint16_t *base, int new_col, int key) {
+        if constexpr (APPEND)
+            if (key == len - 1) return qkv + new_col + h * D + dg;
+        return base + (size_t)key * D;
+    };
     const f16x8 q = *reinterpret_cast<const f16x8 *>(qkv + h * D + dg);
     float m = -INFINITY, l = 0.f, c[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int jc = j0; jc < j1; jc += 8 * NT) {
@@ -213,10 +218,10 @@ __global__ __launch_bounds__(64 * NW) void k_attn_decode(uint16_t *__restrict__ 
         f16x8 kr[NT], vr[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            if (t < nt) kr[t] = *reinterpret_cast<const f16x8 *>(kb + (size_t)min(jc + slot + 8 * t, j1 - 1) * D);
+            if (t < nt) kr[t] = *reinterpret_cast<const f16x8 *>(row(kb, E, min(jc + slot + 8 * t, j1 - 1)));
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            if (t < nt) vr[t] = *reinterpret_cast<const f16x8 *>(vb + (size_t)min(jc + slot + 8 * t, j1 - 1) * D);
+            if (t < nt) vr[t] = *reinterpret_cast<const f16x8 *>(row(vb, 2 * E, min(jc + slot + 8 * t, j1 - 1)));
         float s[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -268,6 +273,29 @@ __global__ __launch_bounds__(64 * NW) void k_attn_decode(uint16_t *__restrict__ 
         }
         att[h * D + lane] = f2h(o / L);
     }
+}
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_attn_decode(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
+                                                         const uint16_t *__restrict__ Kc, const uint16_t *__restrict__ Vc,
+                                                         int maxT, StepArg st_arg, int len_imm) {
+    attn_decode_wg<NW, false>(att, qkv, Kc, Vc, maxT, min(len_imm > 0 ? len_imm : st_arg.p() + 1, maxT), blockIdx.x);
+}
+
+// Decode step, fused: appends this position's K and V (head h's 64 values of each) to the cache and
+// attends over [0, pos], reading key/value pos from the qkv row itself.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_attn_decode_append(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
+                                                                uint16_t *Kc, uint16_t *Vc, int maxT, StepArg st_arg) {
+    constexpr int E = GPT2_N_EMBD, D = GPT2_HEAD_DIM;
+    const int h = blockIdx.x, pos = st_arg.p();
+    if ((unsigned)pos >= (unsigned)maxT) return;   // uniform over the grid: nothing to attend
+    if (threadIdx.x < D) {
+        const size_t at = ((size_t)h * maxT + pos) * D + threadIdx.x;
+        Kc[at] = qkv[E + h * D + threadIdx.x];
+        Vc[at] = qkv[2 * E + h * D + threadIdx.x];
+    }
+    attn_decode_wg<NW, true>(att, qkv, Kc, Vc, maxT, pos + 1, h);
 }
 
 // ------------------------------------------------------------------ KV cache writes
@@ -370,6 +398,11 @@ void attn_decode(uint16_t *att, const uint16_t *qkv, const uint16_t *K, const ui
                  int len_imm) {
     hipLaunchKernelGGL(k_attn_decode<16>, dim3(GPT2_N_HEAD), dim3(1024), 0, stream(), att, qkv, K, V, maxT, st, len_imm);
     check_launch("k_attn_decode");
+}
+
+void attn_decode_append(uint16_t *att, const uint16_t *qkv, uint16_t *K, uint16_t *V, int maxT, StepArg st) {
+    hipLaunchKernelGGL(k_attn_decode_append<16>, dim3(GPT2_N_HEAD), dim3(1024), 0, stream(), att, qkv, K, V, maxT, st);
+    check_launch("k_attn_decode_append");
 }
 
 void argmax_advance(const uint16_t *logits, int V, int *state, int *tokens, int max_pos) {

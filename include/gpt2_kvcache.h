@@ -70,7 +70,8 @@ typedef struct GPT2DecodeGraph GPT2DecodeGraph;
 GPT2DecodeGraph *gpt2_decode_graph_create(const GPT2Backend *be, const GPT2WeightsGPU *w, GPT2KVCache *kv,
                                           GPT2ScratchGPU *s, gpt2_half *logits, int *tokens);
 /* How the captured step runs:
- *   GPT2_DECODE_MULTI       the step's kernels one after another (49 launches per token; more for other backends);
+ *   GPT2_DECODE_MULTI       the step's kernels one after another (49 launches per token; 62 when a scratch or weight
+ *                           pointer is null, or not 16-byte aligned; more for other backends);
  *   GPT2_DECODE_PERSISTENT  one persistent kernel per token: 256 work-groups run every phase of the
  *                           step and exchange the small activation vectors through coherent
  *                           flag words instead of kernel boundaries.  Needs this library's GEMV

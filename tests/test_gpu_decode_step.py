@@ -1,8 +1,9 @@
-"""The multi-kernel decode step's kernels (csrc/decode_step.hip) against the general sequence (one launch
-per op through the backend's slots), and decode attention against float64 attention.
+"""The multi-kernel decode step's kernels (csrc/decode_step.hip) against the step that buffers they do not take
+run (the LayerNorm, gelu and residual inside the GEMVs), that step on each such kind of buffers, and decode
+attention against float64 attention.
 
-A step takes the general sequence when a buffer is not 16-byte aligned; a copy of one LayerNorm gain at an
-odd address makes the same weights take it.  Both round to fp16 at the same points and differ in the order
+A step leaves the kernels of decode_step.hip when a buffer is not 16-byte aligned; a copy of one LayerNorm
+gain at an odd address makes the same weights do so.  Both round to fp16 at the same points and differ in the order
 of fp32 sums, so logits and cache rows are held to the gates of the persistent step against the
 eager one: rel_err = max|a - b| / max|b| <= 1e-2, KL < 2e-3."""
 import ctypes as C
@@ -32,9 +33,10 @@ def random_cache(pkg, L, kv, pos, seed):
     kv.kv.len = pos
 
 
-def step(pkg, L, gpu, kv, scr, backend, token, pos):
+def step(pkg, L, gpu, kv, scr, backend, token, pos, captures=True):
     logits, caps = pkg.Dev(V * 2), pkg.Dev(14 * E * 2)
-    L.gpt2_decode_step_cuda(pkg.backend(backend), C.byref(gpu), C.byref(kv.kv), token, pos, C.byref(scr.s), logits.ptr, caps.ptr)
+    L.gpt2_decode_step_cuda(pkg.backend(backend), C.byref(gpu), C.byref(kv.kv), token, pos, C.byref(scr), logits.ptr,
+                            caps.ptr if captures else None)
     L.gpt2_sync()
     pkg.check("decode step")
     assert kv.kv.len == pos + 1
@@ -45,6 +47,18 @@ def step(pkg, L, gpu, kv, scr, backend, token, pos):
 
 def rel_err(a, b):
     return float(np.abs(a.astype(np.float64) - b).max() / np.abs(b).max())
+
+
+def kl(got, ref):
+    p, q = (np.exp(x.astype(np.float64) - x.max()) for x in (ref, got))
+    p, q = p / p.sum(), q / q.sum()
+    return float((p * (np.log(p) - np.log(q))).sum())
+
+
+def copied(pkg, gpu):
+    w = pkg.GPT2WeightsGPU()
+    C.memmove(C.byref(w), C.byref(gpu), C.sizeof(w))
+    return w
 
 
 @pytest.mark.parametrize("backend,keep", [("gemv", None), ("int8", None), ("int8", 0), ("int8", 3)])
@@ -63,9 +77,9 @@ def test_step_matches_general_sequence(pkg, L, model, backend, keep):
         for pos in (0, 1, 4, 5, 31, 33, 127, 129, 255, 512, 1000, 1023):
             token = (pos * 7919 + 3) % V
             random_cache(pkg, L, kv, pos, pos)
-            got = step(pkg, L, model.gpu, kv, scr, backend, token, pos)
+            got = step(pkg, L, model.gpu, kv, scr.s, backend, token, pos)
             random_cache(pkg, L, kv, pos, pos)
-            ref = step(pkg, L, general, kv, scr, backend, token, pos)
+            ref = step(pkg, L, general, kv, scr.s, backend, token, pos)
             assert rel_err(got[0], ref[0]) <= 1e-2, pos
             p = np.exp(ref[0].astype(np.float64) - ref[0].max())
             q = np.exp(got[0].astype(np.float64) - got[0].max())
@@ -76,6 +90,74 @@ def test_step_matches_general_sequence(pkg, L, model, backend, keep):
             same[pos] = False
             assert np.array_equal(got[2][:, :, :, same], ref[2][:, :, :, same]), pos   # no other row touched
             assert rel_err(oracle.f16_to_f32(got[2][:, :, :, pos]), oracle.f16_to_f32(ref[2][:, :, :, pos])) <= 1e-2, pos
+    finally:
+        scr.free()
+        kv.free()
+        if backend == "int8":
+            L.gpt2_quant_free(C.byref(model.q))
+            model.q = None
+            model.gpu.q = None
+
+
+@pytest.mark.parametrize("backend", ["gemv", "int8"])
+@pytest.mark.parametrize("kind", ["scratch", "bias", "matrix"])
+def test_step_on_other_buffers(pkg, L, model, kind, backend):
+    """Buffers that decode_step.hip's kernels do not take: a scratch without ln, ao and ff (the step without
+    captures needs none of them), null biases, matrices at odd addresses.  Same gates against the step on buffers
+    that they take; a captured step gives the eager one's bits."""
+    if backend == "int8":
+        model.quantize()
+    ref_w, w, hold = model.gpu, model.gpu, []
+    scr, kv = pkg.Scratch(1), pkg.KVCache(MAXT)
+    bare = pkg.GPT2ScratchGPU()
+    C.memmove(C.byref(bare), C.byref(scr.s), C.sizeof(bare))
+    if kind == "scratch":
+        bare.ln = bare.ao = bare.ff = None
+    elif kind == "bias":
+        zero = pkg.Dev.from_numpy(np.zeros(3072, np.uint16))
+        hold.append(zero)
+        ref_w, w = copied(pkg, model.gpu), copied(pkg, model.gpu)
+        for layer in range(12):
+            for name in ("qkv_b", "attn_proj_b", "fc_b", "proj_b"):
+                setattr(ref_w.layers[layer], name, zero.ptr)
+                setattr(w.layers[layer], name, None)
+    else:
+        w = copied(pkg, model.gpu)
+        q = pkg.GPT2QWeightsGPU()
+        if backend == "int8":
+            C.memmove(C.byref(q), C.byref(model.q), C.sizeof(q))
+            w.q = C.addressof(q)
+        for layer, name, n in ((0, "qkv_w", 2304 * E), (3, "attn_proj_w", E * E), (5, "fc_w", 3072 * E), (11, "proj_w", 3072 * E)):
+            slot = getattr(q.layers[layer], name) if backend == "int8" else None
+            size, src = (n, slot.q) if slot else (2 * n, getattr(w.layers[layer], name))
+            odd = pkg.Dev(size + 16)
+            hold.append(odd)
+            assert L.gpt2_d2d(odd.ptr + 2, src, size) == 0
+            if slot:
+                slot.q = odd.ptr + 2
+            else:
+                setattr(w.layers[layer], name, odd.ptr + 2)
+    try:
+        for pos in (0, 5, 130, 1000, 1023):
+            token = (pos * 7919 + 3) % V
+            random_cache(pkg, L, kv, pos, pos)
+            ref = step(pkg, L, ref_w, kv, scr.s, backend, token, pos)
+            random_cache(pkg, L, kv, pos, pos)
+            got = step(pkg, L, w, kv, bare, backend, token, pos, captures=False)
+            assert rel_err(got[0], ref[0]) <= 1e-2 and kl(got[0], ref[0]) < 2e-3, pos
+            same = np.ones(MAXT, bool)
+            same[pos] = False
+            assert np.array_equal(got[2][:, :, :, same], ref[2][:, :, :, same]), pos   # no other row touched
+            assert rel_err(oracle.f16_to_f32(got[2][:, :, :, pos]), oracle.f16_to_f32(ref[2][:, :, :, pos])) <= 1e-2, pos
+            random_cache(pkg, L, kv, pos, pos)
+            logits, tokens = pkg.Dev(V * 2), pkg.Dev(4 * MAXT)
+            g = L.gpt2_decode_graph_create_mode(pkg.backend(backend), C.byref(w), C.byref(kv.kv), C.byref(bare), logits.ptr,
+                                                tokens.ptr, pkg.DECODE_MULTI)
+            pkg.check("graph")
+            assert L.gpt2_decode_graph_set(g, token, pos) == 0 and L.gpt2_decode_graph_run(g, 1) == 0
+            assert L.gpt2_decode_graph_sync(g, None, None) == 0
+            L.gpt2_decode_graph_destroy(g)
+            assert np.array_equal(oracle.f16_to_f32(logits.numpy(np.uint16, (V,))), got[0]), pos
     finally:
         scr.free()
         kv.free()
