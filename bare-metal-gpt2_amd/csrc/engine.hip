@@ -616,12 +616,24 @@ static bool fused_decode_ok(const GPT2Backend *be) {
            be->layernorm == gpt2_layernorm && be->add == gpt2_add && be->gelu == gpt2_gelu;
 }
 
+// Whether the scratch rows of one token that a step uses at the same time (x, and those that hold StepPart)
+// are apart: the general sequence works on a scratch whose rows share memory where they are never live together.
+static bool step_rows_apart(const GPT2ScratchGPU *s) {
+    const struct { const gpt2_half *p; int n; } rows[] = {{s->x, GPT2_N_EMBD}, {s->fc, GPT2_FFN_DIM}, {s->qkv, GPT2_QKV_DIM},
+                                                          {s->att, GPT2_N_EMBD}, {s->ao, GPT2_N_EMBD}, {s->ff, GPT2_N_EMBD}};
+    for (const auto &a : rows)
+        for (const auto &b : rows)
+            if (&a != &b && a.p < b.p + b.n && b.p < a.p + a.n) return false;
+    return true;
+}
+
 // The step kernels read every matrix, vector, activation and cache row in 16-byte (activations: up to
 // 8-byte) pieces, always add the biases and hold a wave's share of at most 1024 cached keys in registers.
 static bool step_buffers_ok(const GPT2Backend *be, const GPT2WeightsGPU *w, const GPT2KVCache *kv, const GPT2ScratchGPU *s) {
     auto ok = [](const void *p) { return p && aligned16(p); };
     auto mat = [&](const gpt2_half *h, const GPT2QW *q) { return be->gemv_q && q && q->q ? ok(q->q) && q->s : ok(h); };
-    if (kv->maxT > GPT2_N_CTX || !ok(kv->data) || !ok(s->x) || !ok(s->fc) || !ok(s->qkv) || !ok(s->att) || !ok(s->ao) || !ok(s->ff))
+    if (kv->maxT > GPT2_N_CTX || !ok(kv->data) || !ok(s->x) || !ok(s->fc) || !ok(s->qkv) || !ok(s->att) || !ok(s->ao) || !ok(s->ff) ||
+        !step_rows_apart(s))
         return false;
     if (!ok(w->wte) || !ok(w->wpe) || !ok(w->lnf_g) || !ok(w->lnf_b) || !mat(w->wte, w->q ? &w->q->wte : nullptr)) return false;
     for (int L = 0; L < GPT2_N_LAYER; ++L) {
