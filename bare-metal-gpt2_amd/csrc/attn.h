@@ -33,7 +33,8 @@ __device__ __forceinline__ float key_score(const f16x8 q, const f16x8 k, bool on
 }
 
 // The softmax weights of a wave's scores against their maximum m, in place, and their sum l (both the
-// same in every lane).  At least one score is finite.
+// same in every lane).  If no score is above -inf (keys that score -inf, not only absent ones), m is -inf and
+// the weights and l are 0, as if the wave had no keys: another wave's keys may decide.
 template <int NT>
 __device__ __forceinline__ void key_softmax(float (&s)[NT], float &m, float &l) {
     float mx = s[0];
@@ -41,10 +42,11 @@ __device__ __forceinline__ void key_softmax(float (&s)[NT], float &m, float &l) 
     for (int t = 1; t < NT; ++t) mx = fmaxf(mx, s[t]);
     mx = fmaxf(mx, other_slot(mx));
     m = fmaxf(fmaxf(lane_f(mx, 0), lane_f(mx, 16)), fmaxf(lane_f(mx, 32), lane_f(mx, 48)));
+    const float base = m == -INFINITY ? 0.f : m;
     float sum = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        s[t] = __expf(s[t] - m);
+        s[t] = __expf(s[t] - base);
         sum += s[t];
     }
     sum += other_slot(sum);

@@ -231,7 +231,8 @@ __device__ __forceinline__ void attn_decode_wg(uint16_t *__restrict__ att, const
         float mc, lc;
         key_softmax<NT>(s, mc, lc);
         if (jc > j0) {   // a cache longer than one pass: this pass joins the earlier ones
-            const float mn = fmaxf(m, mc), fo = __expf(m - mn), fc = __expf(mc - mn);
+            const float mn = fmaxf(m, mc);
+            const float fo = l != 0.f ? __expf(m - mn) : 0.f, fc = lc != 0.f ? __expf(mc - mn) : 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) c[e] *= fo;
 #pragma unroll

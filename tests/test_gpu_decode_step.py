@@ -189,8 +189,39 @@ def test_step_on_shared_scratch(pkg, L, model, shared):
         kv.free()
 
 
+def test_step_scores_of_minus_infinity(pkg, L, model):
+    """Keys whose score is -inf weigh nothing, whether they fill a wave's share, a split or the whole cache: same bits
+    as keys of the lowest finite scores, whose weights are 0 too.  The q bias makes dim 0 of every query about 60."""
+    b = np.full(2304, np.float16(0))
+    b[:E:D] = 60.0
+    bias, scr, kv = pkg.Dev.from_numpy(b), pkg.Scratch(1), pkg.KVCache(MAXT)
+    w = copied(pkg, model.gpu)
+    for layer in range(12):
+        w.layers[layer].qkv_b = bias.ptr
+    odd = pkg.Dev(2 * E + 32)
+    assert L.gpt2_d2d(odd.ptr + 2, model.gpu.layers[7].ln1_g, 2 * E) == 0
+    other = copied(pkg, w)   # takes the step of fused GEMVs
+    other.layers[7].ln1_g = odd.ptr + 2
+    try:
+        for pos, keys in ((1, (0, 1)), (33, (0, 2)), (33, (9, 18)), (33, (32, 33)), (33, (0, 33)), (200, (8, 24)), (1023, (256, 512))):
+            out = []
+            for low in (np.float16(-np.inf), np.float16(-65504.0)):
+                c = np.full((12, 2, H, MAXT, D), np.float16(np.nan))
+                c[:, :, :, :pos] = np.random.default_rng(pos).standard_normal((12, 2, H, pos, D), dtype=np.float32)
+                c[:, 0, :, keys[0]:keys[1], 0] = low
+                for gpu in (w, other):
+                    assert L.gpt2_h2d(kv.kv.data, c.ctypes.data, c.nbytes) == 0
+                    kv.kv.len = pos
+                    out.append(step(pkg, L, gpu, kv, scr.s, "gemv", 11, pos)[0])
+            assert np.isfinite(out[0]).all(), (pos, keys)
+            assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[3]), (pos, keys)
+    finally:
+        scr.free()
+        kv.free()
+
+
 def test_attn_decode_edges(pkg, L):
-    """Lengths around the 8-key slots, 64-key passes and 16 waves, NaN past the length, peaked scores: against
+    """Lengths around the 8-key slots and 16 waves, NaN past the length, peaked scores: against
     float64 attention on the same fp16 values.  Probabilities and sums are fp32, so the error is the fp16
     rounding of the output (half an ulp, 2^-11 of the value) and fp32 noise below it."""
     rng = np.random.default_rng(5)
@@ -213,3 +244,32 @@ def test_attn_decode_edges(pkg, L):
             assert np.abs(got - ref).max() <= 2.0 ** -11 * np.abs(ref).max() + 1e-5 * np.abs(v[:, :n]).max(), n
     finally:
         kv.free()
+
+
+def test_attn_decode_longer_cache(pkg, L):
+    """A hand-built cache of more than 1024 positions (gpt2_kv_alloc makes none): a wave then joins several passes of
+    64 keys.  Keys that score -inf, a wave's first pass, its second and all but the last key: against float64
+    attention with the same scores."""
+    T = 2048
+    rng = np.random.default_rng(6)
+    arena = pkg.Dev(12 * 2 * H * T * D * 2)
+    kv = pkg.GPT2KVCache(data=arena.ptr, bytes=arena.nbytes, maxT=T, nLayer=12, nHead=H, headDim=D, len=0)
+    k, v = (rng.standard_normal((H, T, D), dtype=np.float32).astype(np.float16) for _ in range(2))
+    q = (2.0 * rng.standard_normal((3 * E,), dtype=np.float32)).astype(np.float16)
+    q[:E:D] = 2.0
+    dq, out = pkg.Dev.from_numpy(q), pkg.Dev(2 * E)
+    for n, low in ((1025, ()), (1100, ()), (2048, ()), (1100, (0, 64)), (1100, (64, 72)), (2048, (0, 2047)), (1100, (72, 400))):
+        kn = k[:, :n].copy()
+        if low:
+            kn[:, low[0]:low[1], 0] = -np.inf
+        plane = np.full((2, H, T, D), np.float16(np.nan))
+        plane[0, :, :n], plane[1, :, :n] = kn, v[:, :n]
+        assert L.gpt2_h2d(arena.at(5 * plane.nbytes), plane.ctypes.data, plane.nbytes) == 0
+        L.gpt2_attn_decode(out.ptr, dq.ptr, C.byref(kv), 5, n)
+        L.gpt2_sync()
+        pkg.check("attn_decode")
+        got = out.numpy(np.float16, (H, D)).astype(np.float64)
+        s = np.einsum("hjd,hd->hj", kn.astype(np.float64), q[:E].reshape(H, D).astype(np.float64)) / 8.0
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        ref = np.einsum("hj,hjd->hd", p / p.sum(axis=1, keepdims=True), v[:, :n].astype(np.float64))
+        assert np.abs(got - ref).max() <= 2.0 ** -11 * np.abs(ref).max() + 1e-5 * np.abs(v[:, :n]).max(), (n, low)
