@@ -24,9 +24,20 @@ constexpr int AF_TILE = AF_CK * 128;            // bytes of a chunk's keys (or v
 [[maybe_unused]] constexpr int AF_RING = 2 * 2 * AF_TILE;   // a wave's two stages of keys and values
 constexpr int AF_T2 = 928;                      // prompts longer than this take two query tiles a block
 
+// Eight halves from p; aligned: p is 16-byte aligned.
+template <bool ALIGNED>
+__device__ __forceinline__ f16x8 load_half8(const uint16_t *p) {
+    f16x8 v;
+    if constexpr (ALIGNED) v = *reinterpret_cast<const f16x8 *>(p);
+    else __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
 // The pointers are __restrict__ parameters of an inlined function, which tells the compiler that the LDS
 // reads below do not alias the direct loads in flight (it would wait for them ahead of every read).
-template <int QT>
+// DIRECT = false takes keys and values through registers, for a qkv that is not 16-byte aligned: direct-to-LDS
+// loads of 16 bytes are only issued at 16-byte aligned addresses.  Same values in the same places, same bits.
+template <int QT, bool DIRECT>
 __device__ __forceinline__ void attn_tiles(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv, int T,
                                            uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc, int maxT, int h, int qb) {
 #if defined(__HIP_DEVICE_COMPILE__)   // LDS address-space pointers exist only in the device pass
@@ -52,12 +63,14 @@ __device__ __forceinline__ void attn_tiles(uint16_t *__restrict__ att, const uin
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const size_t row = (size_t)min(c * AF_CK + 8 * i + lr, T - 1) * S3 + lc;
-            __builtin_amdgcn_global_load_lds(Kb + row, G2_LDS(dst + 1024 * i), 16, 0, 0);
+            if constexpr (DIRECT) __builtin_amdgcn_global_load_lds(Kb + row, G2_LDS(dst + 1024 * i), 16, 0, 0);
+            else *reinterpret_cast<f16x8 *>(dst + 1024 * i + 16 * lane) = load_half8<false>(Kb + row);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const size_t row = (size_t)min(c * AF_CK + 8 * i + lr, T - 1) * S3 + lc;
-            __builtin_amdgcn_global_load_lds(Vb + row, G2_LDS(dst + AF_TILE + 1024 * i), 16, 0, 0);
+            if constexpr (DIRECT) __builtin_amdgcn_global_load_lds(Vb + row, G2_LDS(dst + AF_TILE + 1024 * i), 16, 0, 0);
+            else *reinterpret_cast<f16x8 *>(dst + AF_TILE + 1024 * i + 16 * lane) = load_half8<false>(Vb + row);
         }
     };
 
@@ -70,16 +83,16 @@ __device__ __forceinline__ void attn_tiles(uint16_t *__restrict__ att, const uin
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const uint16_t *Qp = qkv + (size_t)min(q0 + 16 * qt + jq, T - 1) * S3 + h * D;
-        qf[qt][0] = *reinterpret_cast<const f16x8 *>(Qp + 8 * g);
-        qf[qt][1] = *reinterpret_cast<const f16x8 *>(Qp + 32 + 8 * g);
+        qf[qt][0] = load_half8<DIRECT>(Qp + 8 * g);
+        qf[qt][1] = load_half8<DIRECT>(Qp + 32 + 8 * g);
     }
     const int ft = q0 + ((threadIdx.x >> 3) & (QB - 1)), fd = (threadIdx.x & 7) * 8;
     f16x8 fk = {}, fv = {};
     static_assert(64 * AF_W >= QB * 8, "a thread per 16-byte chunk");
     if (Kc) {
         const uint16_t *src = qkv + (size_t)min(ft, T - 1) * S3 + E + h * D + fd;
-        fk = *reinterpret_cast<const f16x8 *>(src);
-        fv = *reinterpret_cast<const f16x8 *>(src + E);
+        fk = load_half8<DIRECT>(src);
+        fv = load_half8<DIRECT>(src + E);
     }
     asm volatile("" ::: "memory");
 
@@ -210,7 +223,7 @@ __device__ __forceinline__ void attn_tiles(uint16_t *__restrict__ att, const uin
 #endif
 }
 
-template <int QT>
+template <int QT, bool DIRECT>
 __global__ __launch_bounds__(64 * AF_W) void k_attn_prefill(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,
                                                             int T, uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc,
                                                             int maxT) {
@@ -230,16 +243,18 @@ __global__ __launch_bounds__(64 * AF_W) void k_attn_prefill(uint16_t *__restrict
         }
     }
     if (qi >= nb) return;                      // the grid is rounded up (whole work-group leaves)
-    attn_tiles<QT>(att, qkv, T, Kc, Vc, maxT, h, nb - 1 - qi);
+    attn_tiles<QT, DIRECT>(att, qkv, T, Kc, Vc, maxT, h, nb - 1 - qi);
 }
 
 // Kc, Vc (optional): the layer's K and V cache planes ([H][maxT][D]), filled with this prompt's rows
 // (the prefill scatter of cuda/kvcache.cu:66-81, done inside the attention launch).
 void attention_prefill(uint16_t *att, const uint16_t *qkv, int T, uint16_t *Kc, uint16_t *Vc, int maxT) {
     static_assert(GPT2_N_HEAD == 12, "the XCD assignment covers 12 heads on 8 XCDs");
-    const int qt = T > AF_T2 ? 2 : 1;
-    hipLaunchKernelGGL(qt == 2 ? k_attn_prefill<2> : k_attn_prefill<1>, dim3(8 * 3 * cdiv(cdiv(T, 16 * qt), 2)),
-                       dim3(64 * AF_W), 0, stream(), att, qkv, T, Kc, Vc, maxT);
+    // gpt2_attention_flash refuses an unaligned qkv; a prefill's own scratch may have one
+    const bool direct = aligned16(qkv);
+    const int qt = direct && T > AF_T2 ? 2 : 1;
+    const auto fn = !direct ? k_attn_prefill<1, false> : qt == 2 ? k_attn_prefill<2, true> : k_attn_prefill<1, true>;
+    hipLaunchKernelGGL(fn, dim3(8 * 3 * cdiv(cdiv(T, 16 * qt), 2)), dim3(64 * AF_W), 0, stream(), att, qkv, T, Kc, Vc, maxT);
     check_launch("k_attn_prefill");
 }
 

@@ -61,3 +61,38 @@ def test_cache_fill_with_attention(pkg, L, synth, T):
         scr.free()
         kv.free()
         m.free()
+
+
+@pytest.mark.parametrize("T", [1, 17, 130, 1000])
+def test_prefill_with_unaligned_qkv_rows(pkg, L, synth, T):
+    """A hand-built scratch whose qkv buffer starts 2 bytes past a 16-byte boundary: keys and values go through
+    registers instead of direct-to-LDS loads; the same logits and cache rows bit for bit as on an aligned scratch.  (The skinny
+    GEMM and the fold want aligned rows of C; both are off here, so that QKV itself has the same bits.)"""
+    m = pkg.Model(synth.make_body(seed=33, plain=False))
+    ids = pkg.Dev.from_numpy(synth.token_ids(T, seed=T))
+    scr, kv = pkg.Scratch(T), pkg.KVCache(1024)
+    odd, rows = pkg.GPT2ScratchGPU(), pkg.Dev(T * 3 * E * 2 + 32)
+    C.memmove(C.byref(odd), C.byref(scr.s), C.sizeof(odd))
+    odd.qkv = rows.ptr + 2
+    logits = pkg.Dev(50257 * 2)
+    caps = pkg.GPT2CapsGPU()
+    caps.logits = logits.ptr
+    out = []
+    L.gpt2_tune_prefill_lnfold(0)
+    L.gpt2_tune_gemm_skinny(0)
+    try:
+        for s in (scr.s, odd):
+            cache = np.full(kv.kv.bytes // 2, 0x3C00, np.uint16)
+            assert L.gpt2_h2d(kv.kv.data, cache.ctypes.data, cache.nbytes) == 0
+            L.gpt2_prefill_fill_cache(pkg.backend("flash"), C.byref(m.gpu), C.byref(kv.kv), ids.ptr, T, C.byref(s), C.byref(caps))
+            L.gpt2_sync()
+            pkg.check("prefill")
+            assert L.gpt2_d2h(cache.ctypes.data, kv.kv.data, cache.nbytes) == 0
+            out.append((logits.numpy(np.uint16, (50257,)), cache.copy()))
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    finally:
+        L.gpt2_tune_prefill_lnfold(-1)
+        L.gpt2_tune_gemm_skinny(-1)
+        scr.free()
+        kv.free()
+        m.free()
