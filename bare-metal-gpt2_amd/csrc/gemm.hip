@@ -1069,10 +1069,14 @@ static int forced_cfg() {
 //         attn-proj M=64 4.3 -> 3.7, 256 4.5 -> 4.1, 512 4.5 -> 4.2
 //         fc M=64 4.5 -> 4.0, 128 5.2 -> 4.4, 320 7.1 -> 5.9, 640 10.7 -> 7.6, 1000 10.9 -> 9.7
 //         mlp-proj M=320 8.3 -> 7.1, 640 13.1 -> 9.1, 1000 13.2 -> 11.5
-//   INT8  QKV M=160 5.2 -> 4.6, 448 6.6 -> 6.1, 896 10.5 -> 8.2, 1000 10.6 -> 9.7
+//   INT8  QKV M=160 5.2 -> 4.6, 448 6.6 -> 6.1, 896 10.2 -> 8.4, 1000 10.2 -> 9.6
 //         attn-proj M=320 4.4 -> 4.2
 //         fc M=320 6.5 -> 6.0, 640 9.0 -> 8.2, 1000 12.5 -> 11.1
 //         mlp-proj M=256 8.3 -> 7.9, 1000 12.3 -> 11.5
+// INT8 QKV keeps its 48x32 tiles to 672 rows, where they are 1008 work-groups, four a CU (656 rows: 7.0, 128x64
+// 8.2).  INT8 mlp-proj's 48x64 tiles take four k groups (53) at 705-768, 833-896 and 961-1024 rows, 12, 14 and 16
+// tiles of rows, which the XCDs share evenly (740 rows: 11.2, two k groups 11.7), and two (36) at 11, 13 and 15
+// (690: 12.3, four 12.9; 800: 12.8, 13.3; 930: 13.1, 13.5).
 // At M in (448, 512] fc keeps its 48x64 tiles: 96x64 ones take 7.2 us alone against 7.7, but the whole
 // P=512 fp16 prefill 597 us against 588.
 struct PickRow {
@@ -1090,8 +1094,12 @@ static const PickRow kPick[] = {
     {448, {{5, 54}, {31, 31}, {26, 35}, {23, 45}}},
     {512, {{35, 35}, {31, 31}, {26, 35}, {23, 45}}},
     {640, {{26, 35}, {36, 36}, {1, 55}, {16, 53}}},
-    {704, {{1, 55}, {36, 36}, {56, 57}, {52, 53}}},
+    {672, {{1, 35}, {36, 36}, {56, 57}, {52, 36}}},
+    {704, {{1, 55}, {36, 36}, {56, 57}, {52, 36}}},
+    {768, {{1, 55}, {36, 36}, {58, 58}, {52, 53}}},
+    {832, {{1, 55}, {36, 36}, {58, 58}, {52, 36}}},
     {896, {{1, 55}, {36, 36}, {58, 58}, {52, 53}}},
+    {960, {{56, 57}, {36, 36}, {58, 58}, {52, 36}}},
     {1024, {{56, 57}, {36, 36}, {58, 58}, {52, 53}}},
 };
 

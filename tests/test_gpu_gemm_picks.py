@@ -6,7 +6,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 SHAPES = {"qkv": (2304, 768), "attn_proj": (768, 768), "fc": (3072, 768), "mlp_proj": (768, 3072)}
-EDGES = (64, 96, 128, 160, 224, 256, 320, 448, 512, 640, 704, 896, 1024)
+EDGES = (64, 96, 128, 160, 224, 256, 320, 448, 512, 640, 672, 704, 768, 832, 896, 960, 1024)
 
 
 @pytest.mark.parametrize("int8", [False, True])
