@@ -278,7 +278,7 @@ __device__ uint64_t g_sk_ws[SK_WS_WORDS];
 // LNP (k_gemm_dl_ln): A is the LayerNorm of X[m0 .. m0+BM) (K = 768, gamma ln_g, beta ln_b), built
 // once per work-group into an LDS panel that holds all of the tile's A; the ring then carries W only.
 // SK > 1 (k_gemm_sk) splits K across SK work-groups per tile (see the split-K state below).
-template <int BN, int BM, int WN, int WM, int S, bool QW, int KS, int U, int EPI, bool LNP, int SK = 1>
+template <int BN, int BM, int WN, int WM, int S, bool QW, int KS, int U, int EPI, bool LNP, int SK = 1, bool STAGED = false>
 __device__ __forceinline__ void gemm_dl(uint16_t *__restrict__ C, const uint16_t *__restrict__ A,
                                         const void *__restrict__ Wv, const float *__restrict__ Ws,
                                         const uint16_t *__restrict__ bias, int M, int N, int K, int tiles_m,
@@ -677,11 +677,49 @@ __device__ __forceinline__ void gemm_dl(uint16_t *__restrict__ C, const uint16_t
     }
     // Epilogue: lane holds D[n][m] for n = nb..nb+3, m = mrow, and stores them as one 8-byte store, whatever the
     // alignment of C's rows (odd N, the tied head's 50257 columns, leaves three rows in four 2, 4 or 6 bytes
-    // past a multiple of 8; the hardware takes such stores).  Staging such tiles through LDS to store whole row
-    // pieces measured the same or slower (1024 x 50257, 768 inputs: 192x128 tiles 121.5 us staged, 118 direct)
-    // and barred tiles larger than the ring; even rows store faster (50256 columns: 107).
+    // past a multiple of 8; the hardware takes such stores).  Even rows store faster (1024 x 50257 against 50256
+    // columns, 768 inputs, 192x128 tiles: 117 us, 109).
     if constexpr (RLN || LNF)
         if (!vec_store) return;   // the host runs the fold only where C rows are 8-byte aligned
+    if constexpr (STAGED) {
+        // STAGED: tiles of such rows go through the idle LDS ring and leave row by row, a wave storing 64
+        // consecutive column pairs (dword-aligned in C; a lone first or last column as a 2-byte store).
+        static_assert(EPI == EPI_NONE && KS == 1 && SK == 1, "the plain one-group form");
+        if (!vec_store) {
+            constexpr int CS = BN + 4;   // staged row stride (halves): rows 8 bytes apart in banks
+            static_assert(BM * CS * 2 <= S * STAGE, "staged C tile fits the LDS ring");
+            uint16_t *ct = reinterpret_cast<uint16_t *>(smem_all);
+            lds_barrier();   // every wave is done with the last k-tile's fragments
+#pragma unroll
+            for (int a = 0; a < TN; ++a) {
+                const int nl = wn0 + a * 16 + lgrp * 4;
+#pragma unroll
+                for (int b = 0; b < TM; ++b) {
+                    uint16_t o[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float v = acc[a][b][i];
+                        if constexpr (QW) v = v * sc_e[a][i];
+                        o[i] = f2h(v + (bias ? h2f((uint16_t)bs_e[a][i]) : 0.f));
+                    }
+                    *reinterpret_cast<uint2 *>(ct + (wm0 + b * 16 + lrow) * CS + nl) =
+                        uint2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+                }
+            }
+            lds_barrier();
+            const int ncols = min(BN, N - n0);
+            for (int r = wave_all; r < BM && m0 + r < M; r += NW) {
+                const uint16_t *src = ct + r * CS;
+                uint16_t *dst = C + (size_t)(m0 + r) * N + n0;
+                const int head = (int)(((uintptr_t)dst >> 1) & 1);   // column 0 is not 4-byte aligned
+                for (int c = head + 2 * lane; c + 1 < ncols; c += 128)
+                    *reinterpret_cast<uint32_t *>(dst + c) = (uint32_t)src[c] | ((uint32_t)src[c + 1] << 16);
+                if (lane == 0 && head) dst[0] = src[0];
+                if (lane == 1 && ((ncols - head) & 1)) dst[ncols - 1] = src[ncols - 1];
+            }
+            return;
+        }
+    }
     if (kg != 0) return;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
@@ -744,6 +782,17 @@ __global__ __launch_bounds__(WN *WM * KS * 64) void k_gemm_dl(uint16_t *__restri
                                                          const uint16_t *resid) {
     gemm_dl<BN, BM, WN, WM, S, QW, KS, U, EPI, false>(C, A, Wv, Ws, bias, M, N, K, tiles_m, ntiles, vec_store, resid,
                                                       nullptr, nullptr, LnFold{});
+}
+
+// k_gemm_dl whose tiles leave through LDS where C's rows are not 8-byte aligned (STAGED).
+template <int BN, int BM, int WN, int WM, int S, bool QW>
+__global__ __launch_bounds__(WN *WM * 64) void k_gemm_dl_staged(uint16_t *__restrict__ C, const uint16_t *__restrict__ A,
+                                                           const void *__restrict__ Wv, const float *__restrict__ Ws,
+                                                           const uint16_t *__restrict__ bias, int M, int N, int K,
+                                                           int tiles_m, int ntiles, int vec_store,
+                                                           const uint16_t *resid) {
+    gemm_dl<BN, BM, WN, WM, S, QW, 1, 1, EPI_NONE, false, 1, true>(C, A, Wv, Ws, bias, M, N, K, tiles_m, ntiles, vec_store,
+                                                                 resid, nullptr, nullptr, LnFold{});
 }
 
 // k_gemm_dl with K split over SK work-groups per tile (grid = tiles x SK): for tiles large enough
@@ -940,9 +989,11 @@ static const GemmCfg kCfgs[] = {
     G2_DCFGUF(96, 128, 2, 4, 4, 1, 2),  // 58: 8 waves, wave tile 48x32 (fc)
     G2_DCFG(192, 128, 4, 2, 2),         // 59: 8 waves, wave tile 48x64, double-buffered (vocabulary-sized N)
     G2_DCFG(128, 128, 4, 2, 2),         // 60: 8 waves, wave tile 32x64, double-buffered (vocabulary-sized N)
+    {128, 64, 64, 64, 512, k_gemm_dl_staged<128, 64, 4, 2, 2, false>, k_gemm_dl_staged<128, 64, 4, 2, 2, true>, G2_NOFUSE,
+     true, "dl_bn128_bm64_w4x2_s2_staged"},   // 61: as 46, odd rows of C through LDS
 };
 static const int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
-static_assert(sizeof(kCfgs) / sizeof(kCfgs[0]) == 61, "the pick table names configs by index");
+static_assert(sizeof(kCfgs) / sizeof(kCfgs[0]) == 62, "the pick table names configs by index");
 
 // Any K % 8 == 0 (int8: K % 16 == 0): predicated loads, one k-tile of prefetch.
 #define G2_GCFG(BN, BM, WN, WM) \
@@ -1103,6 +1154,41 @@ static const PickRow kPick[] = {
     {1024, {{56, 57}, {36, 36}, {58, 58}, {52, 53}}},
 };
 
+// Vocabulary-sized N (the tied head, 50257 rows of W) has many tiles per CU, and what bounds it is what each
+// tile reads through L2 per FLOP: double-buffered tiles of 128 rows of A (60; fp16 from 449 rows on 192x128, 59),
+// unless the last of them would be half empty, where 64-row tiles do less padding (46, 61).  us over three sets of
+// buffers in turn, 768 inputs, 50257 columns, 46 or 61 against the chosen one:
+//   fp16  100 rows 27.0 -> 20.5, 224-256 47.8 -> 43.9, 384 63.2 -> 56.5, 512 81.8 -> 68.2, 777 113 -> 94, 1024 146 -> 117
+//   INT8  100 rows 25.0 -> 18.8, 320 48.6 -> 45.1, 512 77 -> 63.5, 1024 148 -> 114; 192x128 tiles lose there (75 at 512
+//         rows: at 142 registers a lane one work-group fits a CU, not two)
+// The counts, columns and K where the larger tiles lose keep 64 rows a tile:
+//   - between one and a half rounds of the 512 work-groups that the chip holds (fp16, to 256 rows; 36001 columns,
+//     256 rows: 564 tiles 29.1, 64 rows a tile 24.8; but 32771, 100: 257 tiles 15.1, 19.8), or few of them (16384, 384:
+//     18.3, 17.9); 192x128 tiles that end just past a round (16384, 700: 516 tiles 34.9, 60 30.5);
+//   - fp16 rows of C at odd addresses with fewer columns (20001 x 640, 1024 rows: 59 50.7, 60 44.1, 61 45.8; 700: 36.9,
+//     34.6, 34.5; 24577 x 768, 700: 57, 51.8, 45.4);
+//   - fp16, K < 384 to 512 rows (50257 x 192, 512 rows: 59 35.9, 61 32.9; at 384 inputs 44.6, 50.0).
+// Odd rows of 64-row tiles are stored directly (46) or through LDS (61).  Through LDS is faster in fp16 where the last
+// tile is about half full or more (50257 columns, 192 rows 35.0, direct 36.0; 448 69.3, 70.7; but 129 32.0, 30.6), and
+// everywhere where the rows of C move by 2 bytes against the memory's sectors (49153 columns, 192 rows: fp16 32.8,
+// 37.5, INT8 30.8, 32.6); elsewhere INT8, everything to 64 rows (50257, 64 rows: 16.3, 16.8) and even N (30522, 192
+// rows: 16.7, 17.2) are faster directly.
+static int pick_vocab(int M, int N, int K, bool qw) {
+    const int mt = cdiv(M, 64);   // 64-row tiles; odd: half of the last 128-row tile is padding
+    const long t128 = (long)cdiv(N, 128) * cdiv(M, 128), t192 = (long)cdiv(N, 192) * cdiv(M, 128);
+    const bool odd = N % 4 != 0;
+    if (qw) {
+        if (t128 >= 256 && !(mt % 2 == 1 && mt <= 3)) return 60;
+    } else if (odd && N < 28000) {
+    } else if (mt <= 7) {
+        if (mt % 2 == 0 && N >= 20000 && t128 >= (N % 64 == 1 ? 384 : 256) && (mt > 4 || t128 <= 512 || t128 >= 768)) return 60;
+    } else if (K >= 384 || mt > 8) {
+        return t192 >= 684 || (!odd && t192 >= 384 && t192 <= 512) ? 59 : 60;
+    }
+    const bool full = (M - 1) % 64 >= 28;
+    return N % 2 && (N % 64 == 1 || (!qw && M > 64 && (full || N < 28000))) ? 61 : 46;
+}
+
 static int pick_cfg(int M, int N, int K, bool qw = false) {
     if (forced_cfg() >= 0 && cfg_usable(g_force_cfg, M, N, K)) return g_force_cfg;
     int shape = -1;
@@ -1119,22 +1205,8 @@ static int pick_cfg(int M, int N, int K, bool qw = false) {
         }
     // Other shapes.  Few rows and a long K: four k groups per tile keep more waves busy.
     if (M <= 64 && K >= 2048 && N <= 4096 && cfg_fits(47, K)) return 47;
-    // Vocabulary-sized N (the tied head, 50257 rows of W) has many tiles per CU, and what bounds it is what each
-    // tile reads through L2 per FLOP: double-buffered tiles of 128 rows of A, unless the last of them would be
-    // half empty, where 64-row tiles do less padding.  768 inputs, us, 128x64 tile against the chosen one:
-    //   fp16  65-128 rows 128x128 (100 rows 23.9 -> 18.7), 193-256 and 321-384 too (224: 37.4 -> 35.2, 384: 52.4
-    //         -> 50.0), from 449 on 192x128 (512: 68.5 -> 62.3, 777: 112.6 -> 99.4, 1024: 150.1 -> 118.5; 128x128
-    //         63.8, 104.6, 129.1); 128x64 stays ahead at 160 rows (27.4, 128x128 over 35), 320 (42.2, 44.0) and
-    //         448 (57.4, 60.0)
-    //   INT8  128x128 (100: 24.1 -> 18.7, 320: 46.6 -> 44.0, 512: 73.4 -> 61.8, 1024: 151.4 -> 120.2; 192x128
-    //         there 137.0), 128x64 only to 64 rows (13.9, 17.5) and at 129-192 (160: 30.1, 35.2)
-    // Below one work-group per CU the small tile's count wins (16384 columns, 100 rows: 128 work-groups of 128x128
-    // 11.4 us, 256 of 128x64 8.5; from 256 on 128x128: 16384 x 256 rows 12.9 -> 12.8, INT8 13.5 -> 12.2).
     if (N >= 16384 && M > 32) {
-        const int mt = cdiv(M, 64);   // 64-row tiles; odd: half of the last 128-row tile is padding
-        const bool half = mt % 2 == 1 && mt <= (qw ? 3 : 7);
-        int c = 46;
-        if (!half && (long)cdiv(N, 128) * cdiv(M, 128) >= 256) c = !qw && mt > 7 ? 59 : 60;
+        const int c = pick_vocab(M, N, K, qw);
         if (cfg_fits(c, K)) return c;
     }
     // Otherwise the largest tile that still gives about one work-group per CU (256 CUs), among the

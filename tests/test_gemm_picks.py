@@ -1,4 +1,4 @@
-"""Tile picks between whose ends another tile measured faster (us beside each): the dispatch is host code."""
+"""Tile picks where another tile measured slower (us beside each): the dispatch is host code."""
 import pytest
 
 QKV, MLP = (2304, 768), (768, 3072)
@@ -15,3 +15,16 @@ QKV, MLP = (2304, 768), (768, 3072)
 ])
 def test_trunk_picks(L, shape, int8, rows, cfg):
     assert {L.gpt2_tune_gemm_pick_q(m, *shape, int8) for m in range(rows[0], rows[1] + 1)} == {cfg}
+
+
+@pytest.mark.parametrize("n,k,int8,rows,cfg", [
+    (50257, 768, 0, 192, 61), (50257, 768, 0, 448, 61),   # rows of C through LDS 35.0, directly 36.0; 69.3, 70.7
+    (50257, 768, 0, 129, 46), (50257, 768, 1, 192, 46),   # directly 30.6, through LDS 32.0; 32.3, 34.0
+    (50257, 192, 0, 512, 61),                             # 64 rows a tile 32.9, 192x128 tiles 35.9
+    (24577, 768, 0, 700, 61),                             # 64 rows a tile 45.4, 192x128 tiles 57.0
+    (16384, 768, 0, 700, 60),                             # 128x128 tiles 30.5, 192x128 34.9
+    (36001, 768, 0, 256, 61),                             # 64 rows a tile 24.8, 128x128 tiles 29.1
+    (49153, 768, 1, 192, 61),                             # through LDS 30.8, directly 32.6
+])
+def test_vocabulary_picks(L, n, k, int8, rows, cfg):
+    assert L.gpt2_tune_gemm_pick_q(rows, n, k, int8) == cfg
