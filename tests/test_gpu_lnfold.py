@@ -95,8 +95,10 @@ def assert_close(got, ref, tol=5e-3):
 
 
 @pytest.mark.parametrize("backend", ["flash", "int8"])
-@pytest.mark.parametrize("T", [2, 17, 64, 200, 512, 1024])
+@pytest.mark.parametrize("T", [2, 17, 64, 65, 96, 97, 128, 129, 160, 161, 200, 224, 225, 256, 257, 321, 512, 513, 641, 673,
+                               705, 769, 897, 1024])
 def test_lnfold_matches_unfolded(pkg, L, synth, model, backend, T):
+    """A length in every range of the tile picks, both ends of those where the fold runs by default."""
     ids = synth.token_ids(T, seed=T + 11)
     if backend == "int8":
         model.quantize()
