@@ -67,9 +67,4 @@ __device__ __forceinline__ void reduce_values(float (&c)[8]) {
     for (int e = 0; e < 8; ++e) c[e] = group_sum(c[e] + other_slot(c[e]));
 }
 
-__device__ __forceinline__ void load_q(f16x8 (&q)[8], const uint16_t *qp) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) q[c] = *reinterpret_cast<const f16x8 *>(qp + 8 * c);
-}
-
 }  // namespace g2

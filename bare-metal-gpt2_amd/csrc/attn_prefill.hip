@@ -4,7 +4,7 @@
 //
 // The fragment layout, softmax and results are attn_block's (attn_prefill.h, the block of the persistent
 // prefill).  What differs is how keys and values arrive: by direct-to-LDS loads of whole 128-byte rows,
-// eight rows an instruction, up to two 32-key chunks ahead.  attn_block loads key fragments straight from
+// eight rows an instruction, one 32-key chunk ahead of the one in use.  attn_block loads key fragments straight from
 // qkv, where neighbouring lanes lie 4608 bytes apart and an instruction takes the address unit four times
 // as long; that, not memory, bounded it (6.7 us at 512 queries against 5.0, 10.0 against 6.8 at 777).
 // The 16-byte chunks of a row are XOR-swizzled by the row (by choosing what each lane fetches), so neither
@@ -12,8 +12,8 @@
 // barrier until the waves' states are merged.
 // MI355X, us a launch, one / two tiles of 16 queries a block: T = 256 3.7 / 4.5, 512 5.0 / 5.9, 777 6.8 /
 // 7.8, 896 7.9 / 8.3, 1024 9.5 / 8.9 (from 13.4).  Two tiles halve the key and value bytes per query but also
-// the work-groups; past 928 queries the one-tile blocks no longer fit the chip in a round and a half (two
-// work-groups of 64 KB of LDS a CU) and two tiles win.
+// the work-groups (708 of one tile at 929 queries, 360 of two; the chip holds 512): the two cross between 896 and
+// 1024, and at 928 the one-tile launch takes 8.5 where the two-tile one at 929 takes 8.8.
 #include "attn_prefill.h"
 
 namespace g2 {

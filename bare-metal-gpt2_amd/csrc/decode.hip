@@ -39,18 +39,23 @@
 //     in later launches (kernel boundaries make them visible); this token's attention takes the new
 //     key and value from the exchanged words instead.
 //
-// Numerics follow the multi-kernel fused step: fp16 activations between phases, fp32 inside,
+// Numerics follow the multi-kernel step: fp16 activations between phases, fp32 inside,
 // LayerNorm with biased variance and eps inside the sqrt, gelu_new, scale after the fp32 sum then
 // bias (then residual), online-softmax attention with scale 1/8, greedy argmax over the fp16 logits
 // with the lowest index among equal maxima.
 #include <cmath>
 #include <type_traits>
 
-#include "attn.h"
 #include "common.h"
 #include "decode.h"
 
 namespace g2 {
+
+// One query's 64 halves in registers.
+__device__ __forceinline__ void load_q(f16x8 (&q)[8], const uint16_t *qp) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) q[c] = *reinterpret_cast<const f16x8 *>(qp + 8 * c);
+}
 
 constexpr int PD_G = 256;                          // work-groups (one per CU)
 constexpr int PD_T = 256;                          // threads per work-group (4 waves)

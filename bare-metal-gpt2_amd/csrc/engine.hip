@@ -297,11 +297,11 @@ static void ln_matmul_site(const GPT2Backend *be, bool fused, bool ln_fuse, gpt2
 // cached per device, dropped by gpt2_free_gpu / gpt2_quant_free.  Weights changed in place need
 // gpt2_tune_prefill_lnfold(0) or a fresh upload.
 //
-// By default the fold runs where it measured faster (interleaved A/B of the whole prefill, fold on
-// against off, MI355X): T <= 128 for both weight formats (7-13% faster), INT8 up to T = 256 (4-5%).
-// Past that the fold's per-tile costs (the partials' loads and the producer's extra stores in every
-// work-group) outgrow the two LayerNorm launches it removes per layer: even at T = 384-512, 0.97-0.92
-// at T = 768-1024.
+// By default the fold runs up to T = 128 (whole prefill, interleaved A/B on MI355X: 6-10% faster with it, both
+// weight formats), INT8 up to T = 256 (3-5%).  fp16 loses 3-5% at 129-256.  With
+// the present tiles it would gain again at 257-320 (fp16 4-5%, INT8 3-4%) and 0-2% to 640, where the limits, set
+// with earlier tiles, leave it off; at 768-1024 it is level or 1% slower: its per-tile costs (the partials' loads,
+// the producer's extra stores) then outgrow the two LayerNorm launches a layer.
 static int g_lnfold = -1;       // gpt2_tune_prefill_lnfold: -1 default (by T), 0 off, 1 on at every T > 1
 static int g_lnfold_sites = 0;  // sites that ran folded in the last forward (test hook)
 

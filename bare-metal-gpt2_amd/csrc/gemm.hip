@@ -923,7 +923,7 @@ struct GemmCfg {
      true, "sk_bn" #BN "_bm" #BM "_w" #WN "x" #WM "_s" #S "_u" #U "_x" #SK, SK}
 static const GemmCfg kCfgs[] = {
     G2_DCFGF(96, 64, 2, 4, 4),      // 0: 8 waves, wave tile 48x16
-    G2_DCFGF(128, 64, 4, 2, 3),     // 1: 8 waves, wave tile 32x32 (vocabulary-sized N; INT8 fc at M=1024)
+    G2_DCFGF(128, 64, 4, 2, 3),     // 1: 8 waves, wave tile 32x32 (fp16 fc, QKV at 513-896 rows)
     G2_DCFGF(32, 64, 1, 4, 4),      // 2: 4 waves, wave tile 32x16
     G2_DCFGF(64, 32, 2, 2, 4),      // 3: 4 waves, wave tile 32x16
     G2_DCFG(96, 64, 2, 2, 6),       // 4: 4 waves, wave tile 48x32
@@ -946,18 +946,18 @@ static const GemmCfg kCfgs[] = {
     G2_DCFGK(128, 64, 4, 2, 3, 2),  // 21: two k groups of 8 waves
     G2_DCFGU(48, 32, 3, 2, 4, 2, 2),  // 22: as 15, two k-tiles per barrier
     G2_DCFGUF(48, 32, 3, 2, 6, 2, 2), // 23: as 15, two k-tiles per barrier, 6 stages (mlp-proj)
-    G2_DCFGU(48, 32, 3, 2, 4, 1, 2),  // 24: as 9, two k-tiles per barrier (QKV)
-    G2_DCFGUF(48, 32, 3, 2, 6, 1, 2), // 25: as 9, two k-tiles per barrier, 6 stages (attn-proj)
+    G2_DCFGU(48, 32, 3, 2, 4, 1, 2),  // 24: as 9, two k-tiles per barrier
+    G2_DCFGUF(48, 32, 3, 2, 6, 1, 2), // 25: as 9, two k-tiles per barrier, 6 stages
     G2_DCFGUF(48, 64, 3, 4, 4, 1, 2), // 26: as 20, two k-tiles per barrier (fc)
     G2_DCFGU(48, 64, 3, 4, 6, 1, 2),  // 27: as 20, two k-tiles per barrier, 6 stages
     G2_DCFGU(48, 32, 3, 2, 6, 1, 3),  // 28: as 9, three k-tiles per barrier
     G2_DCFGU(48, 64, 3, 4, 6, 1, 3),  // 29: as 20, three k-tiles per barrier
     G2_DCFGU(48, 32, 3, 2, 6, 2, 3),  // 30: as 15, three k-tiles per barrier
-    G2_DCFGUF(48, 32, 3, 2, 8, 1, 4), // 31: as 9, four k-tiles per barrier (INT8 attn-proj)
+    G2_DCFGUF(48, 32, 3, 2, 8, 1, 4), // 31: as 9, four k-tiles per barrier (attn-proj; fp16 QKV, fc)
     G2_DCFGU(48, 64, 3, 4, 8, 1, 4),  // 32: as 20, four k-tiles per barrier
-    G2_DCFGUF(48, 32, 3, 2, 8, 2, 4), // 33: as 15, four k-tiles per barrier (160 KB of LDS; INT8 mlp-proj)
+    G2_DCFGUF(48, 32, 3, 2, 8, 2, 4), // 33: as 15, four k-tiles per barrier (160 KB of LDS)
     G2_DCFGUF(48, 64, 3, 2, 4, 1, 2),   // 34: 6 waves, wave tile 16x32 (each widened INT8 fragment feeds 2 MFMAs)
-    G2_DCFGUF(48, 32, 3, 1, 4, 1, 2),   // 35: 3 waves, wave tile 16x32 (INT8 QKV, fc)
+    G2_DCFGUF(48, 32, 3, 1, 4, 1, 2),   // 35: 3 waves, wave tile 16x32 (QKV; INT8 fc)
     G2_DCFGUF(48, 64, 3, 2, 4, 2, 2),   // 36: two k groups of 6 waves, wave tile 16x32
     G2_DCFGU(96, 64, 3, 2, 4, 1, 2),    // 37: 6 waves, wave tile 32x32
     G2_DCFGUF(48, 32, 3, 1, 8, 2, 4),   // 38: two k groups of 3 waves, 8 stages, 4 k-tiles per barrier
@@ -1026,8 +1026,9 @@ static const int kNumLnCfgs = (int)(sizeof(kLnCfgs) / sizeof(kLnCfgs[0]));
 
 // The LayerNorm fold's kernels, on the configs the pick table gives each role: the residual GEMMs
 // (attn-proj, mlp-proj: EPI_RESID_LN) and the GEMMs after a LayerNorm (QKV: EPI_LNF, fc:
-// EPI_LNF_GELU), fp16 and INT8 weights, every M range.  A call whose picked config has no entry here (a
-// forced config) runs the LayerNorm launch and the plain GEMM instead.
+// EPI_LNF_GELU), fp16 and INT8 weights, every M range (beyond the lengths where the fold runs by default,
+// lnfold_wanted, for gpt2_tune_prefill_lnfold).  A call whose picked config has no entry here (a forced config)
+// runs the LayerNorm launch and the plain GEMM instead.
 typedef void (*GemmLnfFn)(uint16_t *, const uint16_t *, const void *, const float *, const uint16_t *, int, int, int,
                           int, int, int, const uint16_t *, LnFold);
 struct GemmLnfEntry {
@@ -1111,7 +1112,9 @@ static int forced_cfg() {
 // Measured picks for the GPT-2 trunk shapes, by prompt length: each shape's 12 layer GEMMs (distinct
 // weights) back to back on MI355X, every config of the table at 20 lengths from 33 to 1000, fp16 and INT8
 // weights.  Shapes QKV, attn-proj, fc, mlp-proj; {fp16, INT8}.  Every config that the prefill picks for
-// attn-proj, fc and mlp-proj carries the fused-epilogue kernels (gelu, residual).
+// attn-proj, fc and mlp-proj carries the fused-epilogue kernels (gelu, residual).  attn-proj's tile at 321-512
+// rows (31) takes 4.0 alone where the one before (25) took 4.3; inside the prefill and inside the 48 GEMMs of a
+// forward the two are level (512 rows: 557 and 559 us, 322 and 321).
 // What decides is the number of work-groups: a launch takes about as long for 130 tiles as for 256 (one per
 // CU) and half again as long for 270, so the limits below lie where a tile's count passes 256, and the
 // largest tile (fewest L2 bytes per FLOP) that still gives most CUs one wins; k groups keep its waves busy.

@@ -246,11 +246,12 @@ typedef void (*SkinnyFn)(uint16_t *, const uint16_t *, const void *, const float
 static const SkinnyFn kSkinny[2][2][5] = {{G2_SKN(768, false), G2_SKN(768, true)},
                                           {G2_SKN(3072, false), G2_SKN(3072, true)}};
 
-// Rows of A up to which the skinny kernel takes the trunk shapes.  Measured on MI355X (interleaved
-// A/B of the whole prefill against the tile pipeline and the LayerNorm fold): INT8 weights 1.27x at
-// T = 8, 1.24x at 16, 1.11x at 24-32, 1.04-1.07x at 40-48, level at 64; fp16 1.12x at 8-16, 1.05-1.07x
-// at 24-32, 0.96x at 40 and 0.94x at 64 -- there the fold, which removes the LayerNorm launches,
-// beats the skinny kernel's LayerNorm prologue.  gpt2_tune_gemm_skinny overrides both (0: never).
+// Rows of A up to which the skinny kernel takes the trunk shapes.  Whole prefill on MI355X, interleaved A/B,
+// tiles with the LayerNorm fold over the skinny kernel with its prologue: INT8 weights 1.38 at T = 8, 1.36 at
+// 16, 1.20 at 24-32, 1.13 at 40-48, 1.07 at 64, 1.03 at 80, 0.86 at 96; fp16 1.32 at 8-16, 1.22 at 24-32, 1.13 at
+// 40-48, 1.10 at 64, 1.04 at 80, 0.93 at 96.  The limits are lower than those crossings: they were set when
+// the kernel took its operands as fragments from memory (fp16 then lost from 40 rows on).
+// gpt2_tune_gemm_skinny overrides both (0: never).
 static int g_skinny_max = -1;    // -1: the measured default per weight format
 static int g_skinny_calls = 0;   // launches so far (test hook)
 int skinny_max_m(bool qw) { return g_skinny_max >= 0 ? g_skinny_max : (qw ? 64 : 32); }

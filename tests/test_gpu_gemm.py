@@ -100,8 +100,8 @@ def test_trunk_shapes_every_m_bucket(pkg, L, kind, M):
 @pytest.mark.parametrize("kind", ["fp16", "int8"])
 @pytest.mark.parametrize("M,N,K", [(300, 777, 768), (129, 257, 256), (64, 1001, 192), (512, 2305, 768)])
 def test_unaligned_c_rows(pkg, L, kind, M, N, K):
-    """Odd N (rows of C not 8-byte aligned) with C itself offset by 0, 1 or 3 elements: the tile is
-    staged through LDS and written as dword column pairs plus lone end columns; the elements right
+    """Odd N (rows of C not 8-byte aligned) with C itself offset by 0, 1 or 3 elements: 8-byte
+    stores at whatever 2-byte alignment a row has, lone columns at the end; the elements right
     before and after C must stay untouched."""
     rng = np.random.default_rng(M + N + K)
     A, W, b = f16v(rng, (M, K), 1.0), f16v(rng, (N, K), 0.02), f16v(rng, N, 0.01)
@@ -162,7 +162,7 @@ def test_generic_path_unaligned_a(pkg, L):
 
 def test_every_tile_config(pkg, L):
     """Every tile config on shapes whose K it accepts (K % (64*depth) == 0), ragged M and N, odd N
-    (C rows not 8-byte aligned: the staged epilogue), plus shapes no config accepts (the guarded
+    (C rows not 8-byte aligned: unaligned stores, or through LDS in the staged config), plus shapes no config accepts (the guarded
     kernel)."""
     rng = np.random.default_rng(11)
     for M, N, K in [(100, 200, 136), (512, 768, 768), (7, 300, 768), (77, 130, 3072), (33, 96, 64),
@@ -292,7 +292,7 @@ def test_fused_epilogues(pkg, L, kind, M, N, K):
     """The prefill's fused-epilogue GEMMs (forward_cuda.cu:99-105 folded into the GEMM: gelu_new of
     fp16(A.W^T + b), and fp16(resid + fp16(A.W^T + b)) with resid == C in place and in a separate
     buffer) against the oracle's matmul, gelu and add on the same fp16 values, at the trunk shapes,
-    ragged M, and N with and without 8-byte C rows (the staged epilogue).  Bar as above.  The residual
+    ragged M, and N with and without 8-byte C rows.  Bar as above.  The residual
     form needs 8-byte C rows (it reads the residual 4 columns at a time): elsewhere it declines and
     launches nothing, and the prefill runs the unfused sequence."""
     rng = np.random.default_rng(M * 7 + N + K)
