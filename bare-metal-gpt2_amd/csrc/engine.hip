@@ -619,11 +619,12 @@ static bool fused_decode_ok(const GPT2Backend *be) {
 // Whether the scratch rows of one token that a step uses at the same time (x, and those that hold StepPart)
 // are apart: the general sequence works on a scratch whose rows share memory where they are never live together.
 static bool step_rows_apart(const GPT2ScratchGPU *s) {
-    const struct { const gpt2_half *p; int n; } rows[] = {{s->x, GPT2_N_EMBD}, {s->fc, GPT2_FFN_DIM}, {s->qkv, GPT2_QKV_DIM},
-                                                          {s->att, GPT2_N_EMBD}, {s->ao, GPT2_N_EMBD}, {s->ff, GPT2_N_EMBD}};
+    const struct { uintptr_t at; size_t bytes; } rows[] = {
+        {(uintptr_t)s->x, 2 * GPT2_N_EMBD},   {(uintptr_t)s->fc, 2 * GPT2_FFN_DIM}, {(uintptr_t)s->qkv, 2 * GPT2_QKV_DIM},
+        {(uintptr_t)s->att, 2 * GPT2_N_EMBD}, {(uintptr_t)s->ao, 2 * GPT2_N_EMBD},  {(uintptr_t)s->ff, 2 * GPT2_N_EMBD}};
     for (const auto &a : rows)
         for (const auto &b : rows)
-            if (&a != &b && a.p < b.p + b.n && b.p < a.p + a.n) return false;
+            if (&a != &b && a.at < b.at + b.bytes && b.at < a.at + a.bytes) return false;
     return true;
 }
 
