@@ -1220,6 +1220,11 @@ static int pick_cfg(int M, int N, int K, bool qw = false) {
         if (!cfg_fits(c, K)) continue;
         last = c;
         const long t = (long)cdiv(N, kCfgs[c].bn) * cdiv(M, kCfgs[c].bm);
+        // INT8 64x64 tiles (us): one a CU, two k groups of 32x32 wave tiles widen W half as often (500 x 2000 x 2048
+        // 16.3 -> 10.3, 256 x 4096 x 1024 9.4 -> 7.0, 1000 x 1001 x 768 8.0 -> 6.1); just past one a CU, 96x64 tiles
+        // on three CUs in four are faster (1500 x 768 x 3072 30.0 -> 26.3, 700 x 1500 x 1024 12.1 -> 10.9).
+        if (qw && c == 5 && t > 256) return 0;
+        if (qw && c == 5 && t == 256 && cfg_fits(54, K)) return 54;
         if (t >= 256) return c;
     }
     return last;

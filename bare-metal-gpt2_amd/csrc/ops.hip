@@ -193,7 +193,7 @@ __global__ void k_add8(f16x8 *__restrict__ x, const f16x8 *__restrict__ y, size_
 // Decode attention: one work-group per head, NW waves split the keys [0, len) (attn.h's layout, 64 keys
 // a wave and pass; a cache of 1024 positions is one pass), every load of a pass issued before its first
 // use; the waves' (m, l, c) states meet in LDS.  Bound by latency: a head's 256 KB of keys and values at
-// 1000 positions come through one CU: 5.9 us, 8.8 with a lane per key row (a wave's load then touched 64 rows).
+// 1000 positions come through one CU: 5.5 us, 8.8 with a lane per key row (a wave's load then touched 64 rows).
 // APPEND: the last key and value are the qkv row's own, which the caller is writing to the cache meanwhile.
 template <int NW, bool APPEND>
 __device__ __forceinline__ void attn_decode_wg(uint16_t *__restrict__ att, const uint16_t *__restrict__ qkv,

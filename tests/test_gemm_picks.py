@@ -28,3 +28,12 @@ def test_trunk_picks(L, shape, int8, rows, cfg):
 ])
 def test_vocabulary_picks(L, n, k, int8, rows, cfg):
     assert L.gpt2_tune_gemm_pick_q(rows, n, k, int8) == cfg
+
+
+@pytest.mark.parametrize("n,k,rows,cfg", [
+    (768, 3072, (1345, 1984), 0), (768, 768, (1345, 1984), 0), (1500, 1024, (673, 960), 0),   # 26.3, 64x64 tiles 30.0; 9.1, 10.1; 10.9, 12.1
+    (1001, 768, (961, 1024), 54), (2000, 2048, (449, 512), 54), (4096, 1024, (193, 256), 54),  # 6.1, one k group 8.0; 10.3, 16.3; 7.0, 9.4
+    (4096, 640, (193, 256), 5),   # K not a multiple of 256
+])
+def test_int8_picks_about_one_tile_a_cu(L, n, k, rows, cfg):
+    assert {L.gpt2_tune_gemm_pick_q(m, n, k, 1) for m in rows} == {cfg}

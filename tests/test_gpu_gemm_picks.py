@@ -57,3 +57,24 @@ def test_trunk_gemm_at_pick_edges(pkg, L, shape, int8):
         L.gpt2_sync()
         pkg.check("%s fused M=%d" % (shape, M))
         assert np.array_equal(fused.numpy(np.uint16, (M, N)), add.numpy(np.uint16, (M, N))), M
+
+
+@pytest.mark.parametrize("M,N,K", [(1345, 768, 768), (1350, 768, 3072), (673, 1500, 1024), (961, 1001, 768), (450, 2000, 2048), (193, 4096, 1024)])
+def test_int8_gemm_about_one_tile_a_cu(pkg, L, M, N, K):
+    """INT8 shapes with 256 64x64 tiles or just more, where the tile is picked for the INT8 weights alone: against the
+    float64 product of the same code x scale values, bounds as above; rows past M stay untouched."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.standard_normal((M, K), dtype=np.float32).astype(np.float16)
+    q = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    s = (rng.random(N, dtype=np.float32) + np.float32(0.5)) * np.float32(3e-4)
+    b = (rng.standard_normal(N, dtype=np.float32) * np.float32(0.1)).astype(np.float16)
+    ref = A.astype(np.float64) @ (q * s[:, None].astype(np.float64)).T + b.astype(np.float64)
+    dA, dW, ds, db = (pkg.Dev.from_numpy(x) for x in (A, q, s, b))
+    out = pkg.Dev.from_numpy(np.full((M + 1, N), np.float16(3.0)))
+    L.gpt2_matmul_int8(out.ptr, dA.ptr, dW.ptr, ds.ptr, db.ptr, M, N, K)
+    L.gpt2_sync()
+    pkg.check("int8 gemm")
+    got = out.numpy(np.float16, (M + 1, N))
+    assert (got[M] == 3.0).all()
+    err = np.abs(got[:M].astype(np.float64) - ref)
+    assert (err <= 2.0 ** -11 * np.abs(ref) + 2.0 ** -14 * ref.std()).all(), err.max()
